@@ -656,10 +656,32 @@ int cg_engine_create(const cg_graph* cg, int algorithm, int engine_type, int use
     CG_TRY(e->q_small.ensure(V));
     CG_TRY(e->q_med.ensure(V));
     uint32_t min_chunk = e->opt.chunk_edges;
-    CG_TRY(e->q_chunk.ensure(V + g->E / min_chunk + 2 * kChunkSpread + 1));
+    // narrow frontiers on the GPU schedule run in a level cluster; traces,
+    // profiles and bottom-up min steps are the per-iteration pipeline's
+    const bool cluster = e->opt.sched_mode == CG_SCHED_GPU && !e->partial && !e->opt.trace_path && !e->opt.profile &&
+                         !e->opt.min_pull && !e->opt.fault_flags && V > 0;
+    size_t chunk_slots = V + g->E / min_chunk + 2 * kChunkSpread + 1, cl_bytes = 0;
+    const uint32_t groups = cluster_groups(g->E);
+    if (cluster) {
+      chunk_slots = (chunk_slots + 15) / 16 * 16;
+      // room for four times an even share of any frontier, and for what LDS holds
+      const uint64_t share = 4 * cluster_entry_bound(V, g->E) / groups + kClusterLds;
+      e->cl_cap = (uint32_t)std::min<uint64_t>(share, kClusterSegment);
+      cl_bytes = 2 * sizeof(ClusterCtl) + 2 * (size_t)e->cl_cap * groups * sizeof(ClusterEntry);
+      if (algorithm == CG_SSSP && e->opt.sssp_delta) cl_bytes += 2 * sizeof(uint64_t) * (size_t)kClusterFar * groups;
+    }
+    CG_TRY(e->q_chunk.ensure(chunk_slots + cl_bytes / sizeof(uint64_t)));
+    if (cluster) {
+      e->cl_ctl = reinterpret_cast<ClusterCtl*>(e->q_chunk.p + chunk_slots);
+      e->cl_groups = groups;
+      CG_TRY(launch_fill_u32(reinterpret_cast<uint32_t*>(e->cl_ctl), 0u, 2 * sizeof(ClusterCtl) / 4, e->stream));
+    }
     CG_TRY(e->st.ensure(2));
     CG_TRY(e->hst.ensure(3));
-    CG_TRY(e->hst_map.ensure(3, hipHostMallocMapped | hipHostMallocCoherent));  // two iterations, query done
+    // two iterations, query done, the level cluster's record
+    CG_TRY(e->hst_map.ensure(4, hipHostMallocMapped | hipHostMallocCoherent));
+    static_assert(sizeof(ClusterRecord) <= sizeof(DevStats), "the record takes a statistics slot");
+    std::memset(e->hst_map.p + 3, 0, sizeof(DevStats));
     e->hst_map_dev = e->hst_map.device_ptr();
     if (!e->hst_map_dev) return set_error(CG_ERR_HIP, "mapped statistics buffer has no device address");
     CG_TRY(e->acc.ensure(kAccSlots));

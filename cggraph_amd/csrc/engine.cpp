@@ -45,6 +45,24 @@ constexpr unsigned long long kBfsTailEdges = 256;
 // expansions queued after it launched with at most kTailGrid workgroups
 constexpr unsigned long long kTailEdges = 1ull << 21;
 constexpr uint32_t kTailGrid = 2048;
+// level cluster: largest out-degree of a graph whose first frontier it takes,
+// and the iterations the wide pipeline keeps after a frontier turned out too
+// wide for it
+constexpr uint64_t kClusterRootDegree = 64;
+constexpr uint32_t kClusterBackoff = 8;
+
+// Whether the cluster should take the frontier two iterations after one of m
+// out-edges, the one before it having had prev_m: the frontiers shrink, and
+// at that rate the one it gets fits a level of it.  An iteration of the wide
+// SSSP / CC pipeline costs at least 25 us, so any such tail pays (R-MAT of
+// 10^6 vertices: five iterations); one of BFS costs 8-10 us, as much as the
+// cluster's launch, so the tail must be long: shrinking slowly.
+bool cluster_tail(int alg, unsigned long long m, unsigned long long prev_m) {
+  if (!prev_m || m > prev_m) return false;
+  const double r = (double)m / (double)prev_m;
+  if (alg == CG_BFS && r < 0.5) return false;
+  return (double)m * r * r <= (double)kClusterEdges;
+}
 
 double ms_since(clk::time_point t0) {
   return std::chrono::duration<double, std::milli>(clk::now() - t0).count();
@@ -203,6 +221,25 @@ int wait_stats(cg_engine* e, int slot, uint32_t it) {
     return set_error(CG_ERR_INTERNAL, "statistics of iteration %u were not published", it);
   std::memcpy(&e->hst_last, h, sizeof(DevStats));
   e->hst_last.iter = it;
+  return CG_OK;
+}
+
+// Waits for the level cluster's record of this launch, like wait_stats.
+int wait_cluster(cg_engine* e, ClusterRecord* r) {
+  ClusterRecord* h = e->cl_rec(e->hst_map.p);
+  const uint32_t tag = e->cl_seq;
+  const auto t0 = clk::now();
+  for (uint32_t spin = 1;; ++spin) {
+    if (__atomic_load_n(&h->tag, __ATOMIC_ACQUIRE) == tag) break;
+    __builtin_ia32_pause();
+    if ((spin & 1023) == 0 && ms_since(t0) > 50.0) {
+      CG_HIP(hipStreamSynchronize(e->stream));
+      if (__atomic_load_n(&h->tag, __ATOMIC_ACQUIRE) != tag)
+        return set_error(CG_ERR_INTERNAL, "the level cluster published no record");
+      break;
+    }
+  }
+  std::memcpy(r, h, sizeof(*r));
   return CG_OK;
 }
 
@@ -472,7 +509,11 @@ int engine_run(cg_engine* e, uint32_t root, cg_run_stats* rs) {
   // A run that failed part-way can leave queued-ahead kernels on the stream;
   // drain them before the host resets the statistics records they publish
   // into (their error, if any, was reported by that run).
-  if (!e->clean_end && stream_wait(s) != hipSuccess) (void)hipGetLastError();
+  if (!e->clean_end) {
+    if (stream_wait(s) != hipSuccess) (void)hipGetLastError();
+    if (e->cl_groups)
+      CG_TRY(launch_fill_u32(reinterpret_cast<uint32_t*>(e->cl_ctl), 0u, 2 * sizeof(ClusterCtl) / 4, s));
+  }
   e->clean_end = false;
   e->epoch = (e->epoch + 1) & 0xFFu;
   if (!e->epoch) e->epoch = 1;
@@ -572,6 +613,14 @@ int engine_run(cg_engine* e, uint32_t root, cg_run_stats* rs) {
   // in-edges (built once per graph, kept with it)
   const bool cc_pull1 = fused && alg == CG_CC && !partial && g.E > 0;
   if (cc_pull1) CG_TRY(build_transpose(&g));
+  // Narrow frontiers of the GPU schedule run in the level cluster
+  // (cluster.hpp).  It takes the first frontier of a graph whose frontiers
+  // are narrow throughout -- no more edges than one level may hold, or no
+  // vertex of a degree that widens a frontier at once (lattices, roads) --
+  // and elsewhere the tail of the traversal, once the frontiers shrink.
+  const bool cluster = e->cl_groups && early && mode == CG_SCHED_GPU;
+  const bool cluster_first =
+      cluster && (g.E <= kClusterEdges || (alg != CG_CC && e->caller_g->max_outdeg <= kClusterRootDegree));
   {
     TraverseInit ti{};
     ti.val = e->val.p;
@@ -598,7 +647,7 @@ int engine_run(cg_engine* e, uint32_t root, cg_run_stats* rs) {
     // and the initialisation does iteration 1's front work
     ti.bfs_cnt = early_bfs ? e->bfs_cnt.p : nullptr;
     ti.off = dg.off;
-    ti.bfs_first = early_bfs ? 1 : 0;
+    ti.bfs_first = early_bfs && !cluster_first ? 1 : 0;
     ti.E = g.E;
     ti.bins = fbins;
     ti.q_small = e->q_small.p;
@@ -717,14 +766,88 @@ int engine_run(cg_engine* e, uint32_t root, cg_run_stats* rs) {
   // learned schedule: the choice the previous record made for this
   // iteration (-1: the GPU rule)
   int pending = -1;
-  if (run_ahead && !early_bfs) CG_TRY(enqueue(1));
+  auto launch_cluster_at = [&](uint32_t k0) -> int {
+    ClusterJob j{};
+    j.off = dg.off;
+    j.dst = dg.dst;
+    const int wb = dg.w8 ? 1 : (dg.w16 ? 2 : 4);
+    j.w = wb == 1 ? (const void*)dg.w8 : (wb == 2 ? (const void*)dg.w16 : (const void*)dg.w);
+    j.val = e->val.p;
+    j.bm[0] = e->bm[0].p;
+    j.bm[1] = e->bm[1].p;
+    j.words = words;
+    j.q[0] = e->cl_q();
+    j.q[1] = j.q[0] + (size_t)e->cl_cap * e->cl_groups;
+    j.cap = e->cl_cap;
+    j.far[0] = e->cl_far();
+    j.far[1] = delta ? e->cl_far() + (size_t)kClusterFar * e->cl_groups : nullptr;
+    j.k0 = k0;
+    j.max_edges = kClusterEdges;
+    j.hub_degree = hub_on ? e->opt.hub_degree : 0;
+    j.delta = delta;
+    j.threshold = threshold;
+    j.rs = e->run_state.p;
+    j.st = e->st.p;
+    j.bfs_cnt = alg == CG_BFS ? e->bfs_cnt.p : nullptr;
+    if (++e->cl_seq == 0) e->cl_seq = 2;  // never 0, and its parity alternates
+    j.ctl = e->cl_ctl + (e->cl_seq & 1);
+    j.ctl_next = e->cl_ctl + ((e->cl_seq & 1) ^ 1);
+    j.host_out = e->cl_rec(e->hst_map_dev);
+    j.tag = e->cl_seq;
+    return launch_cluster(alg, wb, j, e->cl_groups, s);
+  };
+  // Takes the cluster's record: its levels are iterations it + 1 .. it +
+  // levels.  *done: the traversal is complete; otherwise the wide pipeline is
+  // queued again from the frontier handed back.
+  uint32_t cl_backoff = 0;  // iterations before the cluster is tried again
+  auto take_cluster = [&](bool* done) -> int {
+    ClusterRecord r{};
+    CG_TRY(wait_cluster(e, &r));
+    local.heavy_iterations += r.levels;
+    local.gpu_vertices += r.verts;
+    local.edges_relaxed += r.edges;
+    local.expand_alg_bytes += 20.0 * (double)r.verts + (alg == CG_SSSP ? 12.0 : 8.0) * (double)r.edges;
+    ++local.expand_launches;
+    m_explored += r.edges;
+    it += r.levels;
+    cur = it & 1;
+    *done = r.n == 0;
+    if (*done) return CG_OK;
+    if (delta) threshold = r.threshold;
+    last_m = ~0ull;
+    prev_m = 0;
+    cl_backoff = kClusterBackoff;
+    if (early_bfs) {
+      bfs_front_q = bfs_step_q = it;
+      bfs_ahead = true;
+      bfs_prev_n = 0;
+    } else {
+      CG_TRY(enqueue(it + 1));
+    }
+    return CG_OK;
+  };
+  bool cl_done = false;
+  bool cl_next = false;  // the cluster takes the frontier after the coming iteration
+  if (cluster_first) {
+    CG_TRY(launch_cluster_at(1));
+    CG_TRY(take_cluster(&cl_done));
+  } else if (run_ahead && !early_bfs) {
+    CG_TRY(enqueue(1));
+  }
+  unsigned long long cl_prev_m = 0;  // frontier edges of the iteration before
   auto tit = clk::now();
   for (;;) {
     ++it;
+    if (cl_done) break;
     const int slot = it & 1;
     DevStats* dst = e->st.p + slot;
     const bool host_now = early_learned && pending >= 0 && decode_choice(pending).host;
-    if (!run_ahead) CG_TRY(enqueue(it));
+    const bool cl_now = cl_next;
+    cl_next = false;
+    if (cl_now) {
+      if (early_bfs) CG_TRY(bfs_queue_upto(it));
+      CG_TRY(launch_cluster_at(it + 1));
+    } else if (!run_ahead) CG_TRY(enqueue(it));
     else if (early_bfs) {
       if (bfs_ahead) CG_TRY(bfs_queue_upto(it + 1));
     } else if (!host_now) {
@@ -759,7 +882,12 @@ int engine_run(cg_engine* e, uint32_t root, cg_run_stats* rs) {
     if (sst.n_active == 0) break;
     prev_m = it > 1 ? last_m : 0;
     last_m = sst.m_active;
-    if (early_bfs) {
+    if (cluster && !cl_now) {
+      if (cl_backoff) --cl_backoff;
+      cl_next = !cl_backoff && cluster_tail(alg, sst.m_active, cl_prev_m) && sst.n_def == 0;
+    }
+    cl_prev_m = sst.m_active;
+    if (early_bfs && !cl_now) {
       if (!bfs_ahead) {
         CG_TRY(bfs_queue_upto(it));
         if (bfs_front_q < it + 1) CG_TRY(bfs_front(it + 1));
@@ -851,6 +979,7 @@ int engine_run(cg_engine* e, uint32_t root, cg_run_stats* rs) {
     // the network's choice for the next iteration, made from this frontier
     pending = (learned && mlp_dev && probs_usable(sst)) ? sst.choice : -1;
     cur ^= 1;
+    if (cl_now) CG_TRY(take_cluster(&cl_done));
   }
   // The query's last pass, queued behind the iterations (those queued past
   // the empty frontier find nothing to do): the TEPS numerator -- BFS on the

@@ -6,6 +6,7 @@
 #include <string>
 #include <vector>
 
+#include "cluster.hpp"
 #include "host_team.hpp"
 #include "kernels.hpp"
 #include "sched.hpp"
@@ -49,6 +50,18 @@ struct cg_engine {
   cg::DevBuf<unsigned long long> bfs_cnt;  // BFS first-visit counters, two parities
   cg::DevBuf<uint32_t> val_snap;       // probe mode: state restored between choices
   cg::DevBuf<uint64_t> bm_snap;
+
+  // level cluster (GPU schedule), behind the chunk queue in q_chunk: two
+  // control blocks used in turn, the entry queues, the far lists of bucketed
+  // runs; its record lies behind the statistics in hst_map.  cl_groups == 0:
+  // this engine does not use it.
+  uint32_t cl_groups = 0, cl_cap = 0, cl_seq = 0;
+  cg::ClusterCtl* cl_ctl = nullptr;
+  cg::ClusterEntry* cl_q() const { return reinterpret_cast<cg::ClusterEntry*>(cl_ctl + 2); }
+  unsigned long long* cl_far() const {
+    return reinterpret_cast<unsigned long long*>(cl_q() + 2 * (size_t)cl_cap * cl_groups);
+  }
+  cg::ClusterRecord* cl_rec(cg::DevStats* stats) const { return reinterpret_cast<cg::ClusterRecord*>(stats + 3); }
 
   // host-team traffic
   cg::DevBuf<uint32_t> d_share_vals, d_cand_id, d_cand_val;
