@@ -28,17 +28,28 @@
 // of cg_batch_run runs the same queries one per engine launch for
 // comparison.
 //
+// Queries whose frontiers are narrow do not take part in the levels: a
+// 2048^2 lattice alone drags every other query through its 4500 levels at
+// 20 us.  Level clusters (cluster.hpp) run them root to end, one launch for
+// all, beside the engines and the levels.  52 queries, four on each of R-MAT
+// s14-s22 and lattices of 256^2-2048^2: 126 -> 71 ms, the cluster launch 41
+// ms of it; with every query of the 512-query set off the engines 328 -> 215
+// ms; with the s18-s22 queries on engines that set is bound by the engine
+// thread and stays at 237 ms.
+//
 // The relaxation is the reference's (my_project/CGgraph/device_algorithm.cuh:
 // 51-54 BFS, 253-257 SSSP), so each query ends at its unique fixed point,
 // bit-identical to a single-query run.
 #include <algorithm>
 #include <chrono>
+#include <cmath>
 #include <memory>
 #include <mutex>
 #include <string>
 #include <thread>
 #include <vector>
 
+#include "cluster.hpp"
 #include "engine.hpp"
 
 namespace cg {
@@ -401,7 +412,9 @@ __global__ void k_batch_advance(BatchState* __restrict__ bs, uint32_t levels) {
   if (threadIdx.x == 0 && blockIdx.x == 0) bs->base += levels;
 }
 
-__global__ void k_batch_reached(const QueryDesc* __restrict__ qd, int q, unsigned long long* __restrict__ acc) {
+// TEPS numerator of every query: blockIdx.y picks the query.
+__global__ void k_batch_reached(const QueryDesc* __restrict__ qd, unsigned long long* __restrict__ acc) {
+  const uint32_t q = blockIdx.y;
   const QueryDesc& Q = qd[q];
   unsigned long long sum = 0;
   for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < Q.V;
@@ -507,6 +520,20 @@ static int batch_engine(cg_graph* g, int alg, cg_engine** out) {
   return CG_OK;
 }
 
+// Whether one level cluster runs a query on g from its root to its end
+// (cluster.hpp): a graph of narrow frontiers, or one small enough for a
+// sixteenth of the chip to do in well under a millisecond.
+constexpr uint64_t kBatchClusterEdges = 1u << 21;
+static bool batch_on_cluster(const cg_graph* g) {
+  return g->max_outdeg <= kClusterRootDegree || g->E <= kBatchClusterEdges;
+}
+// Its expected time, in some unit: the longest queries are taken first.  A
+// narrow graph of V vertices has levels like the square root of V.
+static double batch_cluster_cost(const cg_graph* g, int alg) {
+  if (g->max_outdeg <= kClusterRootDegree) return (alg == CG_SSSP ? 3.0 : 1.0) * std::sqrt((double)g->V);
+  return 20.0 + (double)g->E / 10000.0;
+}
+
 struct EngineQuery {
   cg_engine* e;
   uint32_t root;
@@ -572,8 +599,9 @@ int run_batched(cg_graph* const* graphs, const int* algs, const uint32_t* roots,
     if (roots[i] >= graphs[i]->V) return set_error(CG_ERR_INVALID, "query %d: root %u >= V", i, roots[i]);
     CG_TRY(graphs[i]->ensure_device());
   }
-  // the queries engines run (jq, in order) and those the batch runs (bq)
-  std::vector<int> bq, jq;
+  // the queries engines run (jq, in order), those level clusters run (cq,
+  // longest first) and those that advance level by level together (bq)
+  std::vector<int> bq, jq, cq;
   std::vector<EngineQuery> jobs;
   for (int i = 0; i < nq; ++i) {
     if (batch_on_engine(graphs[i], min_v)) {
@@ -581,6 +609,8 @@ int run_batched(cg_graph* const* graphs, const int* algs, const uint32_t* roots,
       CG_TRY(batch_engine(graphs[i], algs[i], &e));
       jobs.push_back(EngineQuery{e, roots[i], nullptr});
       jq.push_back(i);
+    } else if (batch_on_cluster(graphs[i])) {
+      cq.push_back(i);
     } else {
       bq.push_back(i);
     }
@@ -597,7 +627,10 @@ int run_batched(cg_graph* const* graphs, const int* algs, const uint32_t* roots,
       o += graphs[jq[k]]->V;
     }
   }
-  const int nb = (int)bq.size();
+  const int nb = (int)bq.size(), nc = (int)cq.size();
+  std::stable_sort(cq.begin(), cq.end(), [&](int a, int b) {
+    return batch_cluster_cost(graphs[a], algs[a]) > batch_cluster_cost(graphs[b], algs[b]);
+  });
   // the graph each batched query runs on, its root there, and the map back
   std::vector<cg_graph*> qgraph(nb);
   std::vector<uint32_t> qroot(nb);
@@ -618,16 +651,72 @@ int run_batched(cg_graph* const* graphs, const int* algs, const uint32_t* roots,
   hipStream_t s = nullptr;
   CG_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
   std::unique_ptr<std::remove_pointer<hipStream_t>::type, decltype(&hipStreamDestroy)> sguard(s, hipStreamDestroy);
-  // per-query device arrays: values, stamps and two frontier queues
+  // level clusters: values and two bitmaps per query, queues per cluster.  A
+  // few queries get 16 workgroups each, many get 4, so that more run at once;
+  // half of the chip is left to the engines and the level loop.
+  const uint32_t cgroups = nc <= 8 ? 16 : (nc <= 32 ? 8 : 4);
+  const uint32_t clusters = std::min<uint32_t>((uint32_t)nc, (jobs.empty() && !nb ? 256u : 128u) / cgroups);
+  DevBuf<uint32_t> cval;
+  DevBuf<uint64_t> cbm, cq_mem;
+  std::vector<uint64_t> cpre(nc + 1, 0), wpre(nc + 1, 0);
+  for (int k = 0; k < nc; ++k) {
+    const uint64_t V = graphs[cq[k]]->V;
+    cpre[k + 1] = cpre[k] + (V + 31) / 32 * 32;
+    wpre[k + 1] = wpre[k] + 2 * ((V + 63) / 64);
+  }
+  // the level loop: values, stamps and two frontier queues per query
   std::vector<uint64_t> vpre(nb + 1, 0);
   for (int k = 0; k < nb; ++k) vpre[k + 1] = vpre[k] + qgraph[k]->V;
   const uint64_t totalV = vpre[nb];
   // the batch indexes its items (vertex slots of all queries) with 32 bits
-  if (totalV > 0xFFFFFFFFull)
+  uint64_t slots_v = totalV;
+  for (int i : cq) slots_v += graphs[i]->V;
+  if (slots_v > 0xFFFFFFFFull)
     return set_error(CG_ERR_INVALID, "the batch holds %llu vertex slots over its queries; at most 2^32 - 1",
-                     (unsigned long long)totalV);
+                     (unsigned long long)slots_v);
+  hipStream_t cs = nullptr;
+  std::unique_ptr<std::remove_pointer<hipStream_t>::type, decltype(&hipStreamDestroy)> csguard(nullptr, hipStreamDestroy);
+  ClusterBatch cb{};
+  if (nc) {
+    CG_HIP(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
+    csguard.reset(cs);
+    CG_TRY(cval.ensure(cpre[nc]));
+    CG_TRY(cbm.ensure(wpre[nc]));
+    std::vector<ClusterQuery> hcq(nc);
+    bool bucketed = false;
+    for (int k = 0; k < nc; ++k) {
+      const cg_graph* g = graphs[cq[k]];
+      const uint32_t delta = algs[cq[k]] == CG_SSSP ? opt.sssp_delta : 0;
+      bucketed = bucketed || delta;
+      hcq[k] = ClusterQuery{g->d_off.p, g->d_dst.p, g->has_w ? g->d_w.p : nullptr, cval.p + cpre[k], cbm.p + wpre[k],
+                            ((uint64_t)g->V + 63) / 64, algs[cq[k]], roots[cq[k]], delta};
+    }
+    // control blocks, counters, queries, queue entries and far lists in one allocation
+    const size_t ctl_b = clusters * sizeof(ClusterCtl), q_b = (nc * sizeof(ClusterQuery) + 127) / 128 * 128;
+    const size_t ent_b = (size_t)clusters * 2 * cgroups * kClusterSegment * sizeof(ClusterEntry);
+    const size_t far_b = bucketed ? (size_t)clusters * 2 * cgroups * kClusterFar * sizeof(uint64_t) : 0;
+    CG_TRY(cq_mem.ensure((ctl_b + 128 + q_b + ent_b + far_b) / sizeof(uint64_t)));
+    char* m = reinterpret_cast<char*>(cq_mem.p);
+    cb.ctl = reinterpret_cast<ClusterCtl*>(m);
+    cb.next = reinterpret_cast<uint32_t*>(m + ctl_b);
+    cb.levels = cb.next + 1;
+    cb.q = reinterpret_cast<const ClusterQuery*>(m + ctl_b + 128);
+    cb.entries = reinterpret_cast<ClusterEntry*>(m + ctl_b + 128 + q_b);
+    cb.far = reinterpret_cast<unsigned long long*>(m + ctl_b + 128 + q_b + ent_b);
+    cb.nq = (uint32_t)nc;
+    cb.groups = cgroups;
+    cb.cap = kClusterSegment;
+    CG_HIP(hipMemcpyAsync(m + ctl_b + 128, hcq.data(), nc * sizeof(ClusterQuery), hipMemcpyHostToDevice, cs));
+    CG_TRY(launch_fill_u64(cq_mem.p, 0, (ctl_b + 128) / sizeof(uint64_t), cs));
+    CG_HIP(hipStreamSynchronize(cs));
+  }
   DevBuf<uint32_t> pool;
-  std::vector<QueryDesc> hq(nb);
+  std::vector<QueryDesc> hq(nb + nc);  // the level loop's queries, then (for the reached edges) the clusters'
+  for (int k = 0; k < nc; ++k) {
+    const cg_graph* g = graphs[cq[k]];
+    hq[nb + k] = QueryDesc{g->d_off.p, g->d_dst.p, nullptr, cval.p + cpre[k], nullptr, {nullptr, nullptr}, g->V,
+                           algs[cq[k]], roots[cq[k]], 0, 0, 0};
+  }
   const bool one_kernel = nb <= kLevelMaxQ;
   const size_t level_lds = (3 * (size_t)nb + 1) * sizeof(uint32_t);
   DevBuf<QueryDesc> dq;
@@ -648,13 +737,18 @@ int run_batched(cg_graph* const* graphs, const int* algs, const uint32_t* roots,
                         {b + 2 * (uint64_t)g->V, b + 3 * (uint64_t)g->V}, g->V, alg, qroot[k], delta, hub_deg,
                         hub_delta};
     }
-    CG_TRY(dq.ensure(nb));
+  }
+  if (nb + nc) {
+    CG_TRY(dq.ensure(nb + nc));
+    CG_HIP(hipMemcpyAsync(dq.p, hq.data(), (nb + nc) * sizeof(QueryDesc), hipMemcpyHostToDevice, s));
+    CG_HIP(hipStreamSynchronize(s));
+  }
+  if (nb) {
     CG_TRY(dvpre.ensure(nb + 1));
     CG_TRY(cnt.ensure(3 * (uint64_t)nb));
     CG_TRY(qs.ensure(3 * (uint64_t)nb));
     CG_TRY(item_off.ensure(2 * (uint64_t)nb + 1));  // one kernel per level: the two threshold sets
     CG_TRY(bs.ensure(1));
-    CG_HIP(hipMemcpyAsync(dq.p, hq.data(), nb * sizeof(QueryDesc), hipMemcpyHostToDevice, s));
     CG_HIP(hipMemcpyAsync(dvpre.p, vpre.data(), (nb + 1) * sizeof(uint64_t), hipMemcpyHostToDevice, s));
     CG_HIP(hipStreamSynchronize(s));
 
@@ -705,24 +799,38 @@ int run_batched(cg_graph* const* graphs, const int* algs, const uint32_t* roots,
   std::string wmsg;
   unsigned long long wedges = 0;
   std::thread worker;
+  // the clusters' workgroups first, while the chip is free
+  if (nc) {
+    CG_TRY(launch_fill_u32(cval.p, kUnreached, cpre[nc], cs));
+    CG_TRY(launch_fill_u64(cbm.p, 0, wpre[nc], cs));
+    CG_TRY(launch_cluster_batch(cb, clusters, cs));
+  }
   if (!jobs.empty()) worker = std::thread(run_engine_queries, dev, &jobs, &wrc, &wmsg, &wedges);
   const int brc = nb ? batch_loop() : CG_OK;
   if (worker.joinable()) worker.join();
+  const hipError_t cerr = nc ? hipStreamSynchronize(cs) : hipSuccess;
   const double ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
   if (brc != CG_OK) return brc;
+  if (cerr != hipSuccess) return set_error(CG_ERR_HIP, "batched level clusters: %s", hipGetErrorString(cerr));
   if (wrc != CG_OK) return set_error(wrc, "batched query on an engine: %s", wmsg.c_str());
 
   // TEPS numerator per query and the outputs, outside the timed region
   DevBuf<unsigned long long> acc;
   std::vector<unsigned long long> hacc(64 * 16, 0ull);
-  if (nb) {
+  uint32_t clevels = 0;
+  if (nb + nc) {
     CG_TRY(acc.ensure(64 * 16));
     CG_HIP(hipMemsetAsync(acc.p, 0, 64 * 16 * sizeof(unsigned long long), s));
-    for (int k = 0; k < nb; ++k) {
-      const unsigned bg = (unsigned)std::min<uint64_t>(((uint64_t)hq[k].V + 255) / 256, 2048);
-      hipLaunchKernelGGL(k_batch_reached, dim3(bg ? bg : 1), dim3(256), 0, s, dq.p, k, acc.p);
+    // one launch, or as many as 65 535 rows of workgroups ask for
+    for (int k = 0; k < nb + nc; k += 65535) {
+      const int rows = std::min(nb + nc - k, 65535);
+      uint32_t v = 1;
+      for (int i = k; i < k + rows; ++i) v = std::max(v, hq[i].V);
+      const unsigned bg = std::min<unsigned>((v + 255) / 256, std::max(2048 / rows, 64));
+      hipLaunchKernelGGL(k_batch_reached, dim3(bg, rows), dim3(256), 0, s, dq.p + k, acc.p);
     }
     BATCH_LAUNCH_OK();
+    if (nc) CG_HIP(hipMemcpyAsync(&clevels, cb.levels, sizeof(clevels), hipMemcpyDeviceToHost, s));
     CG_HIP(hipMemcpyAsync(hacc.data(), acc.p, hacc.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
   }
   DevBuf<uint32_t> unmapped;  // values of a renumbered query in the caller's ids
@@ -737,6 +845,9 @@ int run_batched(cg_graph* const* graphs, const int* algs, const uint32_t* roots,
     }
     CG_HIP(hipMemcpyAsync(outs[bq[k]], src, (size_t)hq[k].V * 4, hipMemcpyDeviceToHost, s));
   }
+  for (int k = 0; k < nc && outs; ++k)
+    if (outs[cq[k]])
+      CG_HIP(hipMemcpyAsync(outs[cq[k]], cval.p + cpre[k], (size_t)graphs[cq[k]]->V * 4, hipMemcpyDeviceToHost, s));
   for (size_t k = 0; k < jq.size() && outs; ++k)
     if (outs[jq[k]])
       CG_HIP(hipMemcpyAsync(outs[jq[k]], jslot[k], (size_t)graphs[jq[k]]->V * 4, hipMemcpyDeviceToHost, s));
@@ -744,8 +855,8 @@ int run_batched(cg_graph* const* graphs, const int* algs, const uint32_t* roots,
   if (rs) {
     std::memset(rs, 0, sizeof(*rs));
     rs->ms = ms;
-    rs->iterations = hb.levels_run;
-    rs->expand_launches = replays;
+    rs->iterations = std::max(hb.levels_run, clevels);
+    rs->expand_launches = replays + (nc ? 1 : 0);
     unsigned long long m = wedges;
     for (auto x : hacc) m += x;
     rs->edges_traversed = m;

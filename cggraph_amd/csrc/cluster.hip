@@ -60,19 +60,19 @@ struct ClusterShared {
   uint32_t end[kClusterMaxGroups];
   LevelView view;
   uint32_t id, members;
+  uint32_t query;
+  uint32_t level, list, moves;  // between two traversals of a launch
 };
 
-template <int ALG, class WT>
-__global__ __launch_bounds__(kClusterBlock) void k_cluster(ClusterJob J) {
-  __shared__ ClusterShared S;
-  ClusterCtl* const ctl = J.ctl;
-  const uint32_t t = threadIdx.x, lane = __lane_id(), wv = t / kWave;
-  // ---- registration ----
-  if (t == 0) {
+// Registers the workgroup with a cluster of `want`; false: it came after the
+// registration closed and leaves.
+__device__ __forceinline__ bool cluster_join(ClusterShared& S, ClusterCtl* ctl, uint32_t want) {
+  if (threadIdx.x == 0) {
     uint32_t id = add_agent(&ctl->join, 1u), members = 0;
     if (id == 0) {
+      for (int i = 0; i < 3; ++i) st_agent(&ctl->far[i].min_val, kClusterNone);
       const uint64_t t0 = wall_clock64();
-      while (ld_agent(&ctl->join) < gridDim.x && wall_clock64() - t0 < kJoinTicks) __builtin_amdgcn_s_sleep(1);
+      while (ld_agent(&ctl->join) < want && wall_clock64() - t0 < kJoinTicks) __builtin_amdgcn_s_sleep(1);
       members = __hip_atomic_fetch_or(&ctl->join, kClosed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       st_agent(&ctl->members, members);
     } else if (!(id & kClosed)) {
@@ -83,9 +83,21 @@ __global__ __launch_bounds__(kClusterBlock) void k_cluster(ClusterJob J) {
     S.members = members;
     S.cnt[0] = S.cnt[1] = S.n = S.m = S.stop = S.far_cnt[0] = S.far_cnt[1] = 0;
     S.view = LevelView{};
+    S.level = S.list = S.moves = 0;
   }
   __syncthreads();
-  if (S.id & kClosed) return;  // uniform: came after the registration closed
+  return !(S.id & kClosed);
+}
+
+// One traversal by a cluster.  BATCH: from J.root to its end, whatever the
+// frontiers hold (a queue or list without room leaves its level's frontier to
+// the bitmap, which is then expanded from there); otherwise from the frontier
+// in the bitmap to its end or to a frontier that is handed back, with a record
+// to the host.
+template <int ALG, class WT, bool BATCH>
+__device__ __forceinline__ void cluster_run(ClusterShared& S, const ClusterJob& J) {
+  ClusterCtl* const ctl = J.ctl;
+  const uint32_t t = threadIdx.x, lane = __lane_id(), wv = t / kWave;
   const uint32_t id = S.id, members = S.members;
   const uint32_t nthreads = members * kClusterBlock, gt = id * kClusterBlock + t;
   const uint32_t nwaves = members * kClusterWaves, gw = id * kClusterWaves + wv;
@@ -93,9 +105,9 @@ __global__ __launch_bounds__(kClusterBlock) void k_cluster(ClusterJob J) {
 
   uint32_t nv = 0, stop = 0, m = 0;  // the wavefront's part of the next frontier: vertices
                                      // (wave-uniform), wide pipeline wanted, out-edges (per lane)
-  uint32_t L = 0, F = 0;             // level and far list, counted from the launch's start
   uint32_t e_done = 0, v_done = 0;   // edges and vertices expanded (per lane; SSSP, CC)
-  uint32_t moves = 0;                // redistributions so far
+  // level, far list and redistributions, counted from the launch's start
+  uint32_t L = S.level, F = S.list, moves = S.moves;
 
   // Ends level lvl, which filled the queue of parity qp: the workgroup adds its
   // counts to the level's report and waits until all have.  The queue read in
@@ -294,9 +306,19 @@ __global__ __launch_bounds__(kClusterBlock) void k_cluster(ClusterJob J) {
   uint32_t prev_n = 0;
   unsigned long long edges = 0, verts = 0;
 
-  // ---- the frontier taken over: counted first (one too large is left as it
-  // is), then queued; the other bitmap and the far set are cleared ----
-  {
+  if constexpr (BATCH) {
+    // ---- the root ----
+    if (gw == 0) {
+      if (lane == 0) {
+        st_agent(J.val + J.root, 0u);
+        set_bit(J.bm[(k - 1) & 1], J.root);
+      }
+      push(lane == 0, J.root, 0, J.off[J.root], J.off[J.root + 1] - J.off[J.root], L & 1);
+    }
+    barrier(L, L & 1);
+  } else {
+    // ---- the frontier taken over: counted first (one too large is left as
+    // it is), then queued; the other bitmap is cleared ----
     uint64_t* in = J.bm[(k - 1) & 1];
     uint64_t* out = J.bm[k & 1];
     uint32_t c = 0;
@@ -310,9 +332,6 @@ __global__ __launch_bounds__(kClusterBlock) void k_cluster(ClusterJob J) {
         c += (uint32_t)__popcll(in[i]);
       }
       nv = wave_sum(c);
-    }
-    if (gt == 0) {
-      for (int i = 0; i < 3; ++i) st_agent(&ctl->far[i].min_val, kClusterNone);
     }
     barrier(L++, 0);
     const uint32_t total = S.view.n;
@@ -364,15 +383,16 @@ __global__ __launch_bounds__(kClusterBlock) void k_cluster(ClusterJob J) {
   bool wide = false;
   for (;;) {
     const LevelView V = S.view;
-    if (V.stop || V.m > J.max_edges) {
+    if (!BATCH && (V.stop || V.m > J.max_edges)) {
       wide = true;
       break;
     }
     uint64_t* const bin = J.bm[(k - 1) & 1];
     uint64_t* const bout = J.bm[k & 1];
     const uint32_t qc = L & 1, qp = qc ^ 1;
-    if (V.uneven) redistribute(qc);
-    if (V.n == 0) {
+    const bool by_bitmap = BATCH && V.stop;
+    if (V.uneven && !by_bitmap) redistribute(qc);
+    if (V.n == 0 && !by_bitmap) {
       // bucketed run with nothing near: split the far list
       if (!J.delta) break;
       // (nothing is added to it in this level, so every wavefront reads the same)
@@ -384,7 +404,7 @@ __global__ __launch_bounds__(kClusterBlock) void k_cluster(ClusterJob J) {
         st_agent(&ctl->far[(F + 2) % 3].count, 0u);
         st_agent(&ctl->far[(F + 2) % 3].min_val, kClusterNone);
       }
-      const uint32_t own = S.far_cnt[F & 1];  // at most kClusterFar: a list without room stops the run
+      const uint32_t own = S.far_cnt[F & 1] < kClusterFar ? S.far_cnt[F & 1] : kClusterFar;
       for (uint32_t b = wv * kWave; b < own; b += kClusterBlock) {  // wave-uniform
         const bool in = b + lane < own;
         uint32_t v = 0, x = 0;
@@ -410,25 +430,11 @@ __global__ __launch_bounds__(kClusterBlock) void k_cluster(ClusterJob J) {
       edges += V.m;
       verts += V.n;
       prev_n = V.n;
-      const bool check = V.m > kClusterCheck;
-      const uint32_t tail = S.cnt[qc];
-      uint32_t gs = (tail + kClusterWaves - 1) / kClusterWaves;
-      if (gs > (uint32_t)kWave) gs = kWave;
-      for (uint32_t first = wv * gs; first < tail; first += kClusterWaves * gs) {  // wave-uniform
-        const uint32_t num = tail - first < gs ? tail - first : gs;
-        uint32_t deg = 0, sv = 0, now = 0, first_piece = 0;
-        uint64_t s = 0;
+      // Expands up to 64 entries, one per lane (the first `num`): their edges
+      // spread over the lanes.  now: the vertex's value at present.
+      auto expand = [&](uint32_t num, uint32_t deg, uint32_t sv, uint32_t now, uint64_t s, uint32_t first_piece,
+                        bool check) {
         uint64_t fresh = 0;  // entries whose vertex was not improved again since (it has another entry then)
-        if (lane < num) {
-          const ClusterEntry e = get(qc, first + lane);
-          const uint32_t v = (uint32_t)e.vertex;
-          sv = (uint32_t)(e.vertex >> 32);
-          s = e.row & kMask40;
-          deg = (uint32_t)(e.row >> 48);
-          st_agent(bin + (v >> 6), (uint64_t)0);  // every vertex of the word is in this frontier
-          if constexpr (ALG != CG_BFS) now = ld_agent(J.val + v);
-          first_piece = e.row >> 40 & 1;
-        }
         const uint32_t incl = wave_scan(deg);
         const uint32_t total = lane_value(incl, kWave - 1);
         const uint32_t excl = incl - deg;
@@ -513,11 +519,63 @@ __global__ __launch_bounds__(kClusterBlock) void k_cluster(ClusterJob J) {
             if (ALG == CG_SSSP && J.delta && push_far(far[u], d[u], cand[u], F)) set_bit(bout, d[u]);
           }
         }
+      };
+      if (by_bitmap) {
+        const uint64_t places = (J.words + 7) / 8;
+        for (uint64_t r = 0; r * 8 * nwaves < places; ++r) {  // uniform
+          const uint64_t i = ((r * 8 + lane / 8) * nwaves + wv * members + id) * 8 + lane % 8;
+          uint64_t bits = i < J.words ? ld_agent(bin + i) : 0ull;
+          if (bits) st_agent(bin + i, (uint64_t)0);
+          while (__ballot(bits != 0)) {
+            uint32_t sv = 0, deg = 0;
+            uint64_t s = 0;
+            if (bits) {
+              const uint32_t v = (uint32_t)(i * 64 + (uint64_t)__builtin_ctzll(bits));
+              bits &= bits - 1;
+              s = J.off[v];
+              deg = (uint32_t)(J.off[v + 1] - s);
+              sv = ld_agent(J.val + v);
+            }
+            expand(kWave, deg, sv, sv, s, 0, true);
+          }
+        }
+      }
+      const uint32_t tail = by_bitmap ? 0u : S.cnt[qc];
+      const bool check = V.m > kClusterCheck;
+      uint32_t gs = (tail + kClusterWaves - 1) / kClusterWaves;
+      if (gs > (uint32_t)kWave) gs = kWave;
+      for (uint32_t first = wv * gs; first < tail; first += kClusterWaves * gs) {  // wave-uniform
+        const uint32_t num = tail - first < gs ? tail - first : gs;
+        uint32_t deg = 0, sv = 0, now = 0, first_piece = 0;
+        uint64_t s = 0;
+        if (lane < num) {
+          const ClusterEntry e = get(qc, first + lane);
+          const uint32_t v = (uint32_t)e.vertex;
+          sv = (uint32_t)(e.vertex >> 32);
+          s = e.row & kMask40;
+          deg = (uint32_t)(e.row >> 48);
+          st_agent(bin + (v >> 6), (uint64_t)0);  // every vertex of the word is in this frontier
+          if constexpr (ALG != CG_BFS) now = ld_agent(J.val + v);
+          first_piece = e.row >> 40 & 1;
+        }
+        expand(num, deg, sv, now, s, first_piece, check);
       }
     }
     ++L;
     ++k;
     barrier(L, qp);
+  }
+
+  if constexpr (BATCH) {
+    __syncthreads();  // every wavefront has read the view and the counters kept for the next traversal
+    if (t == 0) {
+      S.level = L + 1;
+      S.list = F;
+      S.moves = moves;
+      if (id == 0) atomicMax(J.batch_levels, k - J.k0);
+    }
+    __syncthreads();
+    return;
   }
 
   // ---- the end ----
@@ -576,7 +634,74 @@ __global__ __launch_bounds__(kClusterBlock) void k_cluster(ClusterJob J) {
   publish(r);
 }
 
+template <int ALG, class WT>
+__global__ __launch_bounds__(kClusterBlock) void k_cluster(ClusterJob J) {
+  __shared__ ClusterShared S;
+  if (cluster_join(S, J.ctl, gridDim.x)) cluster_run<ALG, WT, false>(S, J);
+}
+
+// Batched queries: clusters of b.groups workgroups take queries from the list
+// in order until none is left.
+__global__ __launch_bounds__(kClusterBlock) void k_cluster_batch(ClusterBatch b) {
+  __shared__ ClusterShared S;
+  const uint32_t c = blockIdx.x / b.groups;
+  ClusterCtl* const ctl = b.ctl + c;
+  if (!cluster_join(S, ctl, b.groups)) return;
+  for (uint32_t turn = 1;; ++turn) {
+    // the first workgroup takes the next query; the others wait for its turn
+    if (threadIdx.x == 0) {
+      uint32_t q;
+      if (S.id == 0) {
+        q = add_agent(b.next, 1u);
+        st_agent(&ctl->query, (unsigned long long)turn << 32 | q);
+      } else {
+        unsigned long long x;
+        do {
+          __builtin_amdgcn_s_sleep(2);
+          x = ld_agent(&ctl->query);
+        } while ((x >> 32) != turn);
+        q = (uint32_t)x;
+      }
+      S.query = q;
+    }
+    __syncthreads();
+    const uint32_t qi = S.query;
+    if (qi >= b.nq) return;  // uniform over the cluster
+    const ClusterQuery Q = b.q[qi];
+    ClusterJob J{};
+    J.off = Q.off;
+    J.dst = Q.dst;
+    J.w = Q.w;
+    J.val = Q.val;
+    J.bm[0] = Q.bm;
+    J.bm[1] = Q.bm + Q.words;
+    J.words = Q.words;
+    J.cap = b.cap;
+    J.q[0] = b.entries + (size_t)c * 2 * b.groups * b.cap;
+    J.q[1] = J.q[0] + (size_t)b.groups * b.cap;
+    J.far[0] = b.far + (size_t)c * 2 * b.groups * kClusterFar;
+    J.far[1] = J.far[0] + (size_t)b.groups * kClusterFar;
+    J.k0 = 1;
+    J.root = Q.root;
+    J.delta = Q.delta;
+    J.threshold = Q.delta;
+    J.ctl = ctl;
+    J.batch_levels = b.levels;
+    if (Q.alg == CG_BFS) cluster_run<CG_BFS, uint32_t, true>(S, J);
+    else cluster_run<CG_SSSP, uint32_t, true>(S, J);
+  }
+}
+
 }  // namespace
+
+int launch_cluster_batch(const ClusterBatch& b, uint32_t clusters, hipStream_t s) {
+  if (b.groups < 1 || b.groups > kClusterMaxGroups || !clusters)
+    return set_error(CG_ERR_INTERNAL, "%u clusters of %u workgroups", clusters, b.groups);
+  hipLaunchKernelGGL(k_cluster_batch, dim3(clusters * b.groups), dim3(kClusterBlock), 0, s, b);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return set_error(CG_ERR_HIP, "batched level clusters: %s", hipGetErrorString(e));
+  return CG_OK;
+}
 
 int launch_cluster(int alg, int w_bytes, const ClusterJob& job, uint32_t groups, hipStream_t s) {
   if (groups < 1 || groups > kClusterMaxGroups) return set_error(CG_ERR_INTERNAL, "level cluster of %u workgroups", groups);

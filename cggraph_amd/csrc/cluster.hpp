@@ -87,6 +87,7 @@ struct alignas(128) ClusterFarState {
 struct ClusterCtl {
   alignas(128) uint32_t join;
   alignas(128) uint32_t members;
+  alignas(128) unsigned long long query;     // batches: turn << 32 | query
   alignas(128) uint32_t bar;                 // barriers of a redistribution
   alignas(128) unsigned long long level[3][16];  // level L's report: word [L % 3][0], one per line
   ClusterFarState far[3];                     // far lists, rotating at each split
@@ -118,6 +119,8 @@ struct ClusterJob {
   uint64_t max_edges;
   uint32_t hub_degree;  // a frontier vertex of at least this degree also asks for the wide pipeline (0: off)
   uint32_t delta, threshold;
+  uint32_t root;            // batches: the query's root, and the largest level count so far
+  uint32_t* batch_levels;
   // wide pipeline's state, written when a frontier is handed back
   RunState* rs;
   DevStats* st;
@@ -137,6 +140,33 @@ inline uint32_t cluster_groups(uint64_t E) {
   const uint64_t g = E / 1024;
   return (uint32_t)(g < 1 ? 1 : (g > kClusterMaxGroups ? kClusterMaxGroups : g));
 }
+
+// A batched query for a cluster: every value unreached, bitmaps (2 * words) zero.
+struct ClusterQuery {
+  const uint64_t* off;
+  const uint32_t* dst;
+  const uint32_t* w;
+  uint32_t* val;
+  uint64_t* bm;
+  uint64_t words;
+  int alg;
+  uint32_t root, delta;
+};
+struct ClusterBatch {
+  const ClusterQuery* q;
+  uint32_t nq;
+  uint32_t* next;     // 0: the first query not yet taken
+  uint32_t* levels;   // 0: the largest level count of a query
+  ClusterCtl* ctl;    // one per cluster, zeroed
+  ClusterEntry* entries;     // 2 * groups * cap per cluster
+  unsigned long long* far;   // 2 * groups * kClusterFar per cluster
+  uint32_t groups, cap;
+};
+int launch_cluster_batch(const ClusterBatch& b, uint32_t clusters, hipStream_t s);
+
+// Largest out-degree of a graph whose frontiers are taken to be narrow from
+// any root (lattices, roads).
+constexpr uint64_t kClusterRootDegree = 64;
 
 // One cluster of `groups` workgroups runs job (cluster.hip).  w_bytes: the
 // width of job.w for SSSP.

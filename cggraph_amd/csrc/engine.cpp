@@ -45,10 +45,8 @@ constexpr unsigned long long kBfsTailEdges = 256;
 // expansions queued after it launched with at most kTailGrid workgroups
 constexpr unsigned long long kTailEdges = 1ull << 21;
 constexpr uint32_t kTailGrid = 2048;
-// level cluster: largest out-degree of a graph whose first frontier it takes,
-// and the iterations the wide pipeline keeps after a frontier turned out too
-// wide for it
-constexpr uint64_t kClusterRootDegree = 64;
+// iterations the wide pipeline keeps after a frontier turned out too wide for
+// the level cluster
 constexpr uint32_t kClusterBackoff = 8;
 
 // Whether the cluster should take the frontier two iterations after one of m

@@ -298,10 +298,14 @@ int cg_graph_device_csr(const cg_graph* g, const uint64_t** offsets, const uint3
 /* nq queries (algorithm[i] BFS or SSSP, root[i]) over graph[i]; outs[i] is a
  * host uint32[V_i] buffer or NULL.  mode 0 (batched): the queries on large
  * skewed graphs (opt->batch_engine_v) run one by one on an engine of their
- * graph from a host thread of their own, while all the others advance level
- * by level together, two launches per level, the per-level loop captured in
- * a HIP graph; stats: ms over both, iterations = levels, expand_launches =
- * graph replays, heavy_iterations = queries run on engines, edges_traversed =
+ * graph from a host thread of their own; those on graphs of narrow frontiers
+ * (largest out-degree at most 64) or of at most 2^21 edges run root to end in
+ * one launch whose clusters of workgroups take a query each (batch_block,
+ * batch_grid, batch_levels, batch_group and hub deferral do not apply there);
+ * the others advance level by level together, the per-level loop captured in
+ * a HIP graph.  All three run at once.  stats: ms over all, iterations = the
+ * largest level count, expand_launches = graph replays and cluster launches,
+ * heavy_iterations = queries run on engines, edges_traversed =
  * the TEPS numerator over all queries.  mode 1: one query per engine launch
  * (the comparison path). */
 int cg_batch_run(cg_graph* const* graphs, const int* algorithms, const uint32_t* roots, int nq,

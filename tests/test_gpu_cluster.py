@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 
 import cggraph_amd as cg
+from cggraph_amd import batch
 
 pytestmark = pytest.mark.gpu
 BFS, SSSP, CC = 0, 1, 2
@@ -96,11 +97,9 @@ def test_tails(oracle, scale):
     check(oracle, og, SSSP, roots, sssp_delta=200)
 
 
-@pytest.mark.parametrize("delta", [1, 30])
-def test_full_far_list(oracle, delta):
-    """A bucketed run whose far lists outgrow their room hands back a frontier
-    of waiting vertices only: a hub reaches 200 000 leaves (16 lists hold
-    131 072), each with a chain of its own, all beyond the first bucket."""
+def far_graph(oracle, delta):
+    """A root that reaches 198 000 leaves within three steps, each with a vertex
+    of its own behind it, at weights far beyond a bucket of width delta."""
     leaves, rng = 200_000, np.random.default_rng(delta)
     mid = 5000  # the root's row stays short, so the run starts in the cluster
     src = [np.zeros(50, np.int64), np.repeat(np.arange(1, 51), 60), np.repeat(np.arange(51, 3051), 66)]
@@ -110,4 +109,40 @@ def test_full_far_list(oracle, delta):
     V = mid + 2 * leaves
     og = weighted(oracle, V, np.concatenate(src), np.concatenate(dst), 7)
     og.weight = rng.integers(40, 60_000, og.E).astype(np.uint32)
-    check(oracle, og, SSSP, [0, 60, mid], sssp_delta=delta * 1000)
+    return og, [0, 60, mid]
+
+
+@pytest.mark.parametrize("delta", [1000, 30000])
+def test_full_far_list(oracle, delta):
+    """A bucketed run whose far lists outgrow their room (16 lists hold 131 072
+    entries) hands back a frontier of waiting vertices only."""
+    og, roots = far_graph(oracle, delta)
+    check(oracle, og, SSSP, roots, sssp_delta=delta)
+
+
+@pytest.mark.parametrize("fill", [0, 40])
+def test_batch_on_clusters(oracle, fill):
+    """Batched queries run from root to end on a cluster: lattices, skewed
+    graphs whose frontiers outgrow the queues (with more than 32 queries a
+    cluster has 4 workgroups and room for 32 768 entries) and full far lists
+    (expanded from the bitmap then), beside queries on engines and in the
+    level loop."""
+    far, far_roots = far_graph(oracle, 1000)
+    ogs = [oracle.rmat_graph(16, 16, seed=5, weights=(1, 1000)), oracle.grid_graph(120, 0.1, seed=3), far,
+           oracle.rmat_graph(18, 12, seed=6, weights=(1, 1000))]
+    gs = [cg.Graph.from_csr(o.offsets, o.dest, o.weight) for o in ogs]
+    roots = [[oracle.max_outdeg_vertex(ogs[0]), 7], [0, 7000], far_roots[:2], [oracle.max_outdeg_vertex(ogs[3]), 3]]
+    qs = [(k, a, r) for k in range(4) for a in (BFS, SSSP) for r in roots[k]] + [(1, BFS, 100 + i) for i in range(fill)]
+    for opt in ({"sssp_delta": 0}, {"sssp_delta": 1000}, {"sssp_delta": 3000, "batch_engine_v": 0xFFFFFFFF}):
+        outs, st = batch.run_batch([gs[k] for k, _, _ in qs], [a for _, a, _ in qs], [r for _, _, r in qs], **opt)
+        total = 0
+        for (k, a, r), got in zip(qs, outs):
+            ref = oracle.bfs(ogs[k], r) if a == BFS else oracle.sssp(ogs[k], r)
+            assert np.array_equal(got, ref), (k, a, r, opt)
+            total += oracle.reached_edges(ogs[k], ref)
+        assert st["edges_traversed"] == total
+        on_engines = sum(1 for k, _, _ in qs if ogs[k].V >= 1 << 18 and np.diff(ogs[k].offsets.astype(np.int64)).max() >=
+                         16 * max(-(-ogs[k].E // ogs[k].V), 1))
+        assert on_engines == 8 and st["heavy_iterations"] == (0 if "batch_engine_v" in opt else on_engines)
+    for g in gs:
+        g.close()
