@@ -739,14 +739,16 @@ int cg_engine_run(cg_engine* e, uint32_t root, void* out, cg_run_stats* stats) {
     // point directly; the per-iteration schedulers apply to the frontier
     // engine (directed input, or the heuristic / forced / probe modes).
     DevGraph dg{g.d_off.p, g.d_dst.p, nullptr, nullptr, nullptr, g.V};
+    dg.deg = g.d_deg.p;
     const auto t0 = std::chrono::steady_clock::now();
     if (e->opt.profile) CG_HIP(hipEventRecord(e->ev0, e->stream));
-    st = wcc_hooking(dg, e->val.p, 2, e->stream, nullptr);
+    st = wcc_hooking(dg, e->val.p, e->acc.p, e->stream);
     if (st == CG_OK && e->opt.profile) CG_HIP(hipEventRecord(e->ev1, e->stream));
-    if (st == CG_OK) CG_HIP(hipStreamSynchronize(e->stream));
+    if (st == CG_OK) st = engine_wait(e);
     rs.ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
     if (st == CG_OK && e->opt.profile) {
       float ms = 0;
+      CG_HIP(hipEventSynchronize(e->ev1));
       CG_HIP(hipEventElapsedTime(&ms, e->ev0, e->ev1));
       rs.expand_kernel_ms = ms;
     }

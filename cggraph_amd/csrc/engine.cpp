@@ -1017,6 +1017,15 @@ int engine_run(cg_engine* e, uint32_t root, cg_run_stats* rs) {
   return CG_OK;
 }
 
+int engine_wait(cg_engine* e) {
+  e->epoch = (e->epoch + 1) & 0xFFu;
+  if (!e->epoch) e->epoch = 1;
+  // (the record of the engine's last wait has arrived, so none can land late)
+  __atomic_store_n(&e->hst_map.p[2].iter, 0u, __ATOMIC_RELEASE);
+  CG_TRY(launch_query_done(nullptr, e->hst_map_dev + 2, record_tag(e->epoch, 0), e->stream));
+  return wait_stats(e, 2, 0);
+}
+
 int engine_run_host(cg_engine* e, uint32_t root, cg_run_stats* rs) {
   cg_graph& g = *e->g;
   const uint32_t V = g.V;

@@ -125,6 +125,10 @@ struct cg_engine {
 
 namespace cg {
 int engine_run(cg_engine* e, uint32_t root, cg_run_stats* rs);
+// Waits until every kernel queued on the engine's stream has finished, by
+// polling a record that one more kernel publishes (a stream wait behind short
+// kernels takes 20-25 us).
+int engine_wait(cg_engine* e);
 // The engine without a GPU: every iteration is relaxed by the host team over
 // a host frontier bitmap, on host values (the reference's LIGHT path,
 // CGgraph_engine.cuh:907-912, and the MULTI_CORE engine, GraphNuma.cuh:166-314).

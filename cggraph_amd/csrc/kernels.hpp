@@ -328,8 +328,9 @@ int push_step_from_bitmap(int alg, const DevGraph& g, uint32_t* val, const uint6
                           uint64_t* out, hipStream_t s);
 
 // ---- WCC by hooking (wcc.hip) ----
-int wcc_hooking(const DevGraph& g, uint32_t* parent, uint32_t sample_rounds, hipStream_t s,
-                uint64_t* edges_relaxed);
+// Queues the whole run (parent: the labels); workspace: 16 bytes of device
+// memory.  g needs the degree array.
+int wcc_hooking(const DevGraph& g, uint32_t* parent, void* workspace, hipStream_t s);
 
 // ---- PageRank (pagerank.hip) ----
 struct PrPlan;  // per-graph layout for the pull kernels (tiers, relabelled CSC or source windows)

@@ -10,12 +10,24 @@
 // parent[x] <= x holds throughout, so each tree's root is its minimum id and
 // the final labels equal the label-propagation fixed point bit for bit.
 // The edge order follows Afforest (Sutton, Ben-Nun, Bar, IPDPS'18): link the
-// first `sample_rounds` neighbours of every vertex, compress, find the most
-// frequent root by sampling, then let only vertices outside that component
-// link their remaining edges -- an edge between the large component and
-// another vertex is seen from the other side, because the graph is symmetric.
+// first neighbours of every vertex, compress, find the most frequent root by
+// sampling, then let only vertices outside that component link their
+// remaining edges -- an edge between the large component and another vertex
+// is seen from the other side, because the graph is symmetric.
+//
+// The first neighbour needs no linking: rows are ascending, so parent[v] =
+// min(v, first neighbour) is already a forest of edges of the graph (round 0,
+// fused with the initialisation: no atomics, no reads of other parents).  On
+// skewed graphs that alone leaves almost every vertex in one tree, and the
+// second sampled neighbour -- another line of nearly every row -- is skipped;
+// a lattice, where it leaves many, takes it.  The line: at most 1/8 of the
+// sampled vertices outside the most frequent tree with an edge left to look
+// at, found on the device, so the kernels of the second round are always
+// queued and return at once.  R-MAT s24, 16.8 M vertices, 521 M edges:
+// 0.66 ms of kernels with two linked rounds, 0.39 ms now (0.68 -> 0.42 ms per
+// query with the waits): the first round 275 -> 136 us, the second 183 -> 4 us,
+// compression and the remaining edges 160 -> 223 us, for more of them.
 #include <algorithm>
-#include <vector>
 
 #include "kernels.hpp"
 
@@ -50,7 +62,49 @@ __device__ void link(uint32_t u, uint32_t v, uint32_t* __restrict__ parent) {
   }
 }
 
-__global__ void k_link_round(DevGraph g, uint32_t r, uint32_t* __restrict__ parent) {
+// The root above v, given its parent and grandparent; every step is stored,
+// so the climbs of a long chain's vertices shorten each other.
+__device__ __forceinline__ uint32_t climb(uint32_t v, uint32_t p, uint32_t gp, uint32_t* __restrict__ parent) {
+  while (p != gp) {
+    __hip_atomic_store(parent + v, gp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    p = gp;
+    gp = ld_relaxed(parent + p);
+  }
+  return p;
+}
+
+// Round 0: parent[v] = min(v, first neighbour).  Bound by one line per row
+// (off is streamed); kIlp rows per lane keep that many in flight.
+constexpr int kIlp = 4;
+
+__global__ __launch_bounds__(kBlock) void k_first(DevGraph g, uint32_t* __restrict__ parent) {
+  const uint64_t base = blockIdx.x * (uint64_t)(kBlock * kIlp) + threadIdx.x;
+  uint64_t s[kIlp], e[kIlp];
+  uint32_t d[kIlp];
+#pragma unroll
+  for (int k = 0; k < kIlp; ++k) {
+    const uint64_t v = base + k * kBlock;
+    s[k] = v < g.V ? g.off[v] : 0;
+    e[k] = v < g.V ? g.off[v + 1] : 0;
+  }
+#pragma unroll
+  for (int k = 0; k < kIlp; ++k) d[k] = s[k] < e[k] ? g.dst[s[k]] : 0xFFFFFFFFu;
+#pragma unroll
+  for (int k = 0; k < kIlp; ++k) {
+    const uint64_t v = base + k * kBlock;
+    if (v < g.V) parent[v] = d[k] < (uint32_t)v ? d[k] : (uint32_t)v;
+  }
+}
+
+// What the sampling found: the most frequent root, and how many neighbours of
+// every vertex are linked before the rest (1 or 2).
+struct WccPlan {
+  uint32_t mode, rounds;
+};
+
+__global__ __launch_bounds__(kBlock) void k_link_round(DevGraph g, uint32_t r, const WccPlan* __restrict__ plan,
+                                                       uint32_t* __restrict__ parent) {
+  if (r >= plan->rounds) return;
   for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < g.V;
        v += (uint64_t)gridDim.x * blockDim.x) {
     const uint64_t s = g.off[v], e = g.off[v + 1];
@@ -58,121 +112,151 @@ __global__ void k_link_round(DevGraph g, uint32_t r, uint32_t* __restrict__ pare
   }
 }
 
-__global__ void k_compress(uint32_t V, uint32_t* __restrict__ parent) {
-  for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V;
-       v += (uint64_t)gridDim.x * blockDim.x) {
-    uint32_t p = ld_relaxed(parent + v);
-    uint32_t gp = ld_relaxed(parent + p);
-    while (p != gp) {
-      __hip_atomic_store(parent + v, gp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      p = gp;
-      gp = ld_relaxed(parent + p);
-    }
+// plan: only if that many rounds were linked (NULL: always).
+__global__ __launch_bounds__(kBlock) void k_compress(uint32_t V, uint32_t* __restrict__ parent,
+                                                     const WccPlan* __restrict__ plan, uint32_t rounds) {
+  if (plan && plan->rounds != rounds) return;
+  for (uint64_t base = blockIdx.x * (uint64_t)(kBlock * kIlp) + threadIdx.x; base < V;
+       base += (uint64_t)gridDim.x * (kBlock * kIlp)) {
+    uint32_t p[kIlp], gp[kIlp];
+#pragma unroll
+    for (int k = 0; k < kIlp; ++k) p[k] = base + k * kBlock < V ? ld_relaxed(parent + base + k * kBlock) : 0u;
+#pragma unroll
+    for (int k = 0; k < kIlp; ++k) gp[k] = ld_relaxed(parent + p[k]);
+#pragma unroll
+    for (int k = 0; k < kIlp; ++k)
+      if (base + k * kBlock < V) (void)climb((uint32_t)(base + k * kBlock), p[k], gp[k], parent);
   }
 }
 
-__global__ void k_sample_roots(const uint32_t* __restrict__ parent, uint32_t V, uint64_t seed,
-                               uint32_t n, uint32_t* __restrict__ out) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) {
-    uint64_t z = seed + (uint64_t)(i + 1) * 0x9E3779B97F4A7C15ull;
-    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-    z ^= z >> 31;
-    out[i] = parent[(uint32_t)(z % V)];
-  }
-}
+// The most frequent root among kSamples random vertices (ties to the smaller
+// id) and the number of rounds to link, on the device so the host never
+// waits: one workgroup, each thread counting its sample's occurrences in LDS.
+// Any choice gives the same labels; a good one lets most vertices skip their
+// remaining edges.  rounds: what is linked when it is called; a second call
+// (rounds 2) only looks again if the first asked for that round.  Round 0's
+// trees are climbed here, at most kClimb steps (longer chains, as in a
+// lattice, count as outside and so ask for the second round).
+constexpr int kClimb = 24;
+constexpr uint32_t kSamples = 512;
 
-// The most frequent root among the samples (ties to the smaller id), on the
-// device so the host never waits: one workgroup of kSamples threads, each
-// counting its sample's occurrences in LDS.  Any choice gives the same
-// labels; a good one lets most vertices skip their remaining edges.
-constexpr uint32_t kSamples = 1024;
-
-__global__ __launch_bounds__(kSamples) void k_sample_mode(const uint32_t* __restrict__ samp,
-                                                          uint32_t* __restrict__ mode) {
-  __shared__ uint32_t x[kSamples];
+__global__ __launch_bounds__(kSamples) void k_sample(DevGraph g, const uint32_t* __restrict__ parent, uint64_t seed,
+                                                     uint32_t rounds, WccPlan* __restrict__ plan) {
+  if (rounds == 2 && plan->rounds != 2) return;
+  __shared__ uint4 x4[kSamples / 4];
   __shared__ unsigned long long best[kSamples / 64];
+  __shared__ uint32_t outside;
+  uint32_t* const x = reinterpret_cast<uint32_t*>(x4);
   const uint32_t t = threadIdx.x;
-  x[t] = samp[t];
+  uint64_t z = seed + (uint64_t)(t + 1) * 0x9E3779B97F4A7C15ull;
+  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+  z ^= z >> 31;
+  const uint32_t v = (uint32_t)(z % g.V);
+  const uint64_t deg = g.off[v + 1] - g.off[v];
+  uint32_t mine = parent[v];
+  bool root = false;
+  for (int i = 0; i < kClimb && !root; ++i) {
+    const uint32_t p = parent[mine];
+    root = p == mine;
+    mine = p;
+  }
+  x[t] = mine;
+  if (t == 0) outside = 0;
   __syncthreads();
   uint32_t c = 0;
-  for (uint32_t j = 0; j < kSamples; ++j) c += x[j] == x[t];
+  for (uint32_t j = 0; j < kSamples / 4; ++j) {
+    const uint4 y = x4[j];
+    c += (y.x == mine) + (y.y == mine) + (y.z == mine) + (y.w == mine);
+  }
   // key: larger count first, then smaller id
-  unsigned long long key = ((unsigned long long)c << 32) | (0xFFFFFFFFu - x[t]);
+  unsigned long long key = ((unsigned long long)c << 32) | (0xFFFFFFFFu - mine);
   for (int d = 32; d >= 1; d >>= 1) {
     const unsigned long long o = __shfl_xor(key, d, 64);
     key = o > key ? o : key;
   }
   if (__lane_id() == 0) best[t / 64] = key;
   __syncthreads();
+  key = best[0];
+  for (uint32_t w = 1; w < kSamples / 64; ++w) key = best[w] > key ? best[w] : key;
+  const uint32_t mode = 0xFFFFFFFFu - (uint32_t)(key & 0xFFFFFFFFu);
+  const uint64_t out = __ballot((mine != mode || !root) && deg > rounds);
+  if (__lane_id() == 0) atomicAdd(&outside, (uint32_t)__popcll(out));
+  __syncthreads();
   if (t == 0) {
-    unsigned long long k = best[0];
-    for (uint32_t w = 1; w < kSamples / 64; ++w) k = best[w] > k ? best[w] : k;
-    *mode = 0xFFFFFFFFu - (uint32_t)(k & 0xFFFFFFFFu);
+    plan->mode = mode;
+    plan->rounds = rounds == 2 || outside > kSamples / 8 ? 2 : 1;
   }
 }
 
 // Remaining edges of vertices outside the large component.  A wavefront
-// takes 64 consecutive vertices, tests them one per lane (parent outside the
-// large component, edges left after the sampled ones), then links the rows
-// that need it one at a time with the row spread over the 64 lanes -- most
-// vertices are in the large component or have no edges left, so the test is
-// the bulk of the work and runs 64 wide.
-__global__ __launch_bounds__(kBlock) void k_link_rest(DevGraph g, uint32_t r, const uint32_t* __restrict__ mode,
+// climbs from 256 consecutive vertices, four per lane (compressing as it
+// goes), tests them 64 at a time (root outside the large component, edges
+// left), and each lane links the first kOwnEdges of its
+// own row; what is left of longer rows is linked one row at a time with the
+// row spread over the 64 lanes.  Most vertices are in the large component or
+// have no edges, so the test is the bulk of the work and runs 64 wide; most of
+// the others are leaves below their only neighbour, which a row per wavefront
+// step would take one by one (R-MAT s24 after round 0 alone: 300 us with that,
+// 140 us with the lanes' own edges first, both behind a compression of 91 us;
+// 194 us with the compression in it).
+constexpr int kOwnEdges = 4;
+
+__global__ __launch_bounds__(kBlock) void k_link_rest(DevGraph g, const WccPlan* __restrict__ plan,
                                                       uint32_t* __restrict__ parent) {
-  const uint32_t skip = *mode;
+  const uint32_t skip = plan->mode, r = plan->rounds;
   const uint32_t lane = __lane_id();
-  const uint64_t waves = (uint64_t)gridDim.x * (kBlock / 64);
-  for (uint64_t base = (blockIdx.x * (uint64_t)(kBlock / 64) + threadIdx.x / 64) * 64; base < g.V;
-       base += waves * 64) {
-    const uint64_t v = base + lane;
+  const uint64_t base = (blockIdx.x * (uint64_t)(kBlock / 64) + threadIdx.x / 64) * (64 * kIlp) + lane;
+  uint32_t p[kIlp], gp[kIlp];
+#pragma unroll
+  for (int k = 0; k < kIlp; ++k) p[k] = base + k * 64 < g.V ? ld_relaxed(parent + base + k * 64) : skip;
+#pragma unroll
+  for (int k = 0; k < kIlp; ++k) gp[k] = ld_relaxed(parent + p[k]);
+#pragma unroll
+  for (int k = 0; k < kIlp; ++k)
+    if (base + k * 64 < g.V) p[k] = climb((uint32_t)(base + k * 64), p[k], gp[k], parent);
+#pragma unroll 1
+  for (int k = 0; k < kIlp; ++k) {
+    const uint64_t v = base + k * 64;
     uint64_t s = 0, e = 0;
-    if (v < g.V && ld_relaxed(parent + v) != skip) {
-      s = g.off[v] + r;
+    // the degree array spares the offsets of isolated vertices; a vertex below
+    // its first neighbour was not linked to it by round 0
+    if (v < g.V && p[k] != skip && g.deg[v] != 0) {
+      s = g.off[v];
       e = g.off[v + 1];
+      if (g.dst[s] < (uint32_t)v) s += r;
     }
+#pragma unroll 1
+    for (int i = 0; i < kOwnEdges; ++i)
+      if (s < e) link((uint32_t)v, g.dst[s++], parent);
     for (uint64_t need = __ballot(s < e); need; need &= need - 1) {
       const int l = __builtin_ctzll(need);
       const uint64_t rs = __shfl(s, l, 64), re = __shfl(e, l, 64);
-      for (uint64_t k = rs + lane; k < re; k += 64) link((uint32_t)(base + l), g.dst[k], parent);
+      for (uint64_t x = rs + lane; x < re; x += 64) link((uint32_t)(v - lane + l), g.dst[x], parent);
     }
   }
-}
-
-unsigned grid_of(uint64_t n) {
-  uint64_t b = (n + kBlock - 1) / kBlock;
-  if (b < 1) b = 1;
-  return (unsigned)(b < 65536 ? b : 65536);
 }
 
 }  // namespace
 
-int wcc_hooking(const DevGraph& g, uint32_t* parent, uint32_t sample_rounds, hipStream_t s,
-                uint64_t* edges_relaxed) {
+int wcc_hooking(const DevGraph& g, uint32_t* parent, void* workspace, hipStream_t s) {
   const uint32_t V = g.V;
-  if (edges_relaxed) *edges_relaxed = 0;
   if (V == 0) return CG_OK;
-  CG_TRY(launch_iota_u32(parent, V, s));
-  for (uint32_t r = 0; r < sample_rounds; ++r) {
-    hipLaunchKernelGGL(k_link_round, dim3(grid_of(V)), dim3(kBlock), 0, s, g, r, parent);
-    hipLaunchKernelGGL(k_compress, dim3(grid_of(V)), dim3(kBlock), 0, s, V, parent);
-  }
-  // most frequent root among kSamples samples, found on the device
-  DevBuf<uint32_t> samp;
-  CG_TRY(samp.ensure(kSamples + 1));
-  hipLaunchKernelGGL(k_sample_roots, dim3(kSamples / kBlock), dim3(kBlock), 0, s, parent, V,
-                     (uint64_t)0x5EEDull, kSamples, samp.p);
-  hipLaunchKernelGGL(k_sample_mode, dim3(1), dim3(kSamples), 0, s, samp.p, samp.p + kSamples);
-  const uint64_t waves_grid = std::min<uint64_t>(((uint64_t)V + 255) / 256, 65536);
-  hipLaunchKernelGGL(k_link_rest, dim3((unsigned)(waves_grid ? waves_grid : 1)), dim3(kBlock), 0, s, g,
-                     sample_rounds, samp.p + kSamples, parent);
-  hipLaunchKernelGGL(k_compress, dim3(grid_of(V)), dim3(kBlock), 0, s, V, parent);
+  if (!g.deg) return set_error(CG_ERR_INTERNAL, "component hooking without the degree array");
+  WccPlan* const plan = static_cast<WccPlan*>(workspace);
+  constexpr uint64_t kSeed = 0x5EEDull;
+  const dim3 block(kBlock), rows((unsigned)(((uint64_t)V + kBlock * kIlp - 1) / (kBlock * kIlp)));
+  const dim3 capped(std::min(rows.x, 2048u));  // strides; most often it returns at once
+  hipLaunchKernelGGL(k_first, rows, block, 0, s, g, parent);
+  hipLaunchKernelGGL(k_sample, dim3(1), dim3(kSamples), 0, s, g, parent, kSeed, 1u, plan);
+  hipLaunchKernelGGL(k_compress, capped, block, 0, s, V, parent, plan, 2u);
+  hipLaunchKernelGGL(k_link_round, capped, block, 0, s, g, 1u, plan, parent);
+  hipLaunchKernelGGL(k_compress, capped, block, 0, s, V, parent, plan, 2u);
+  hipLaunchKernelGGL(k_sample, dim3(1), dim3(kSamples), 0, s, g, parent, kSeed, 2u, plan);
+  hipLaunchKernelGGL(k_link_rest, rows, block, 0, s, g, plan, parent);
+  hipLaunchKernelGGL(k_compress, rows, block, 0, s, V, parent, (const WccPlan*)nullptr, 0u);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return set_error(CG_ERR_HIP, "WCC kernels: %s", hipGetErrorString(e));
-  // the sample buffer is freed on return: the kernels reading it end first
-  CG_HIP(hipStreamSynchronize(s));
-  if (edges_relaxed) *edges_relaxed = 0;
   return CG_OK;
 }
 
