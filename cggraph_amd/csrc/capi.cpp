@@ -689,6 +689,19 @@ int cg_engine_create(const cg_graph* cg, int algorithm, int engine_type, int use
     CG_TRY(e->stripes.ensure(kStripeWords));
     CG_TRY(e->run_state.ensure(2));
     if (algorithm == CG_BFS) CG_TRY(e->bfs_cnt.ensure(2 * kBfsCntWords));
+    // label propagation on the queued-ahead pipeline goes bottom-up first
+    // where that pays (a symmetric graph is hooked instead)
+    if (algorithm == CG_CC && !g->symmetric && !e->partial && !e->opt.min_pull && g->E > kClusterEdges &&
+        (e->opt.sched_mode == CG_SCHED_GPU || e->opt.sched_mode == CG_SCHED_LEARNED)) {
+      DevGraph dg{g->d_off.p, g->d_dst.p, nullptr, nullptr, nullptr, g->V};
+      dg.deg = g->d_deg.p;
+      bool pull = false;
+      CG_TRY(cc_source(dg, g->E, &e->cc_z, &pull, e->stream));
+      if (pull) {
+        CG_TRY(e->cc_cnt.ensure(kCcRounds));
+        CG_TRY(e->cc_list.ensure(cc_pull_list_size(g->E)));
+      }
+    }
   }
   if (e->opt.trace_path) {
     e->trace = std::fopen(e->opt.trace_path, "a");

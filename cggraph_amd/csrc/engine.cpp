@@ -658,8 +658,16 @@ int engine_run(cg_engine* e, uint32_t root, cg_run_stats* rs) {
     if (cc_pull1) {
       ti.in_off = g.d_in_off.p;
       ti.in_src = g.d_in_src.p;
+      ti.cc_cnt = e->cc_cnt.p;
     }
     CG_TRY(launch_init_traverse(ti, s));
+    // then bottom-up rounds (ccpull.hip), the frontier they leave in bm[0]
+    if (cc_pull1 && e->cc_cnt.p) {
+      DevGraph cg = dg;
+      cg.in_off = g.d_in_off.p;
+      cg.in_src = g.d_in_src.p;
+      CG_TRY(launch_cc_pull(cg, g.E, e->cc_z, e->val.p, e->bm[0].p, e->cc_cnt.p, e->cc_list.p, s));
+    }
   }
   bool early_timed[4] = {false, false, false, false};
   auto take_timing = [&](int k) -> int {

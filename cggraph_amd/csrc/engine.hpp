@@ -84,6 +84,12 @@ struct cg_engine {
   cg::DevBuf<uint32_t> new_of_d, val_out;
   std::vector<uint32_t> new_of;
 
+  // label propagation: the smallest vertex with out-edges, and the counters
+  // and row list of the bottom-up rounds (cc_cnt.p == NULL: pushes only)
+  uint32_t cc_z = 0;
+  cg::DevBuf<cg::CcPullCounters> cc_cnt;
+  cg::DevBuf<uint32_t> cc_list;
+
   // bottom-up min steps: row of the first in-edge of each edge tile
   cg::DevBuf<uint32_t> pull_tiles;
   bool pull_tiles_ready = false;

@@ -198,6 +198,7 @@ int launch_fused_finish(const StatsPart* parts, uint32_t nparts, uint32_t* strip
 // statistics slots cleared (slot 1's choice -1 when choice1_none), both run
 // states with `visited0`, and -- bfs_cnt not NULL -- the BFS counters with
 // the root's counts in parity 0 (off: the graph's offsets).
+struct CcPullCounters;
 struct TraverseInit {
   uint32_t* val;
   uint64_t V;
@@ -233,6 +234,7 @@ struct TraverseInit {
   // pulled here, and bm0 holds the vertices whose label fell
   const uint64_t* in_off = nullptr;
   const uint32_t* in_src = nullptr;
+  CcPullCounters* cc_cnt = nullptr;  // kCcRounds counters of the bottom-up rounds, cleared
 };
 int launch_init_traverse(const TraverseInit& a, hipStream_t s);
 // BFS under the GPU schedule, two kernels per iteration (traverse.hip): the
@@ -326,6 +328,25 @@ hipError_t stream_wait(hipStream_t s);
 // expansion with scratch queues owned by the caller.
 int push_step_from_bitmap(int alg, const DevGraph& g, uint32_t* val, const uint64_t* in,
                           uint64_t* out, hipStream_t s);
+
+// ---- label propagation, bottom-up rounds (ccpull.hip) ----
+// Counters of one bottom-up round: out-edges of the vertices it changed
+// (striped), rows left to its second kernel.  Zero before the first round.
+constexpr int kCcRounds = 2;                 // queued; the second runs only if the first changed much:
+constexpr unsigned long long kCcShare = 16;  // vertices that send at least 1/16 of the edges
+constexpr int kCcStride = 16;
+struct CcPullCounters {
+  unsigned long long edges[kStripes * kCcStride];
+  uint32_t rows, pad[31];
+};
+// The smallest vertex with out-edges, and whether bottom-up rounds pay: its
+// out-neighbours send at least 1/kCcShare of the edges.  Waits for the stream.
+int cc_source(const DevGraph& g, uint64_t E, uint32_t* z, bool* pull, hipStream_t s);
+uint64_t cc_pull_list_size(uint64_t E);  // entries of the row list
+// kCcRounds rounds on the labels in val; changed_bm: on return the vertices
+// whose out-edges are open (untouched words belong to rounds that did not run).
+int launch_cc_pull(const DevGraph& g, uint64_t E, uint32_t z, uint32_t* val, uint64_t* changed_bm, CcPullCounters* cnt,
+                   uint32_t* list, hipStream_t s);
 
 // ---- WCC by hooking (wcc.hip) ----
 // Queues the whole run (parent: the labels); workspace: 16 bytes of device

@@ -335,6 +335,9 @@ __global__ __launch_bounds__(kBlock) void k_init_traverse(TraverseInit a) {
     a.stripes[i] = (a.minima_empty && i >= (uint64_t)kStripeMinBase) ? 0xFFFFFFFFu : 0u;
   if (a.acc)
     for (uint64_t i = t0; i < (uint64_t)kAccSlots; i += nt) a.acc[i] = 0;
+  if (a.cc_cnt)
+    for (uint64_t i = t0; i < kCcRounds * sizeof(CcPullCounters) / 4; i += nt)
+      reinterpret_cast<uint32_t*>(a.cc_cnt)[i] = 0;
   // BFS: iteration one's direction and queues for frontier {root}, as
   // k_bfs_front decides and compacts them (nothing explored yet, so the push
   // rule reads 15 * deg(root) > E; the chunk size shrinks as for any frontier)
