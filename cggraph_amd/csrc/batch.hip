@@ -522,8 +522,13 @@ static int batch_engine(cg_graph* g, int alg, cg_engine** out) {
 
 // Whether one level cluster runs a query on g from its root to its end
 // (cluster.hpp): a graph of narrow frontiers, or one small enough for a
-// sixteenth of the chip to do in well under a millisecond.
-constexpr uint64_t kBatchClusterEdges = 1u << 21;
+// sixteenth of the chip.  A skewed graph's frontiers outgrow the cluster's
+// queues, which makes each of its levels a walk over the bitmap by sixteen
+// workgroups: seven queries on an R-MAT graph of 2^14 / 2^15 / 2^16 / 2^17
+// vertices (edge factor 16) took 1.1 / 5.7 / 4.1 / 19.0 ms on clusters and
+// 3.4 / 5.0 / 5.3 / 11.6 ms level by level together, so the line lies between
+// the first two.
+constexpr uint64_t kBatchClusterEdges = 1u << 18;
 static bool batch_on_cluster(const cg_graph* g) {
   return g->max_outdeg <= kClusterRootDegree || g->E <= kBatchClusterEdges;
 }

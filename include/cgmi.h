@@ -299,7 +299,7 @@ int cg_graph_device_csr(const cg_graph* g, const uint64_t** offsets, const uint3
  * host uint32[V_i] buffer or NULL.  mode 0 (batched): the queries on large
  * skewed graphs (opt->batch_engine_v) run one by one on an engine of their
  * graph from a host thread of their own; those on graphs of narrow frontiers
- * (largest out-degree at most 64) or of at most 2^21 edges run root to end in
+ * (largest out-degree at most 64) or of at most 2^18 edges run root to end in
  * one launch whose clusters of workgroups take a query each (batch_block,
  * batch_grid, batch_levels, batch_group and hub deferral do not apply there);
  * the others advance level by level together, the per-level loop captured in
