@@ -1,5 +1,5 @@
-// PageRank by pulling over the transposed graph, FP32 with a fixed summation
-// order.
+// PageRank by pulling over the transposed graph, FP32 ranks with a fixed
+// summation order.
 //
 // The reference's PR is not functional (it accumulates into the source on
 // uint32, my_project/CGgraph/device_algorithm.cuh:505-545); only its update
@@ -9,9 +9,8 @@
 //
 // Four layouts, chosen once per graph (the first three pull over the
 // in-edges, the fourth pushes through destination bins):
-//  plain       one sweep over the transposed graph per iteration, rows tiered
-//              by in-degree: one lane / one wavefront per row, and rows of
-//              8192+ in-edges cut into 8192-edge chunks of one workgroup each.
+//  plain       one sweep over the transposed graph per iteration, in blocks of
+//              consecutive rows staged through LDS (row blocks, below).
 //  relabelled  the same sweep over a copy of the CSC whose vertex ids are
 //              renumbered by descending out-degree (ties by id).  On skewed
 //              graphs a small prefix of the ids then carries most edges'
@@ -55,8 +54,18 @@ enum {
 struct PrPlan {
   int layout = kLayoutPlain;
   double stream_bytes = 0;  // per iteration, by design (edge and pair terms + 16 B per vertex)
-  // plain and relabelled pull: tiers over the rows of the CSC in use (one
-  // set per pass; the two-band sweep has two passes)
+  // plain and relabelled pull: blocks of consecutive rows of the CSC in use,
+  // rows of kRowEdges and more in chunks of their own
+  struct RowBlocks {
+    uint32_t n = 0, n_chunks = 0;
+    DevBuf<uint32_t> row;                  // first row of each block (n + 1 entries)
+    DevBuf<uint32_t> long_row;             // the long rows
+    DevBuf<uint32_t> row_chunk, arrived;   // their first chunks (one more entry), chunks done in this sweep
+    DevBuf<uint64_t> chunk_lo, chunk_hi;
+    DevBuf<uint32_t> chunk_of;             // long row of each chunk
+    DevBuf<double> partial;
+  } rows;
+  // two-band sweep: tiers over the rows of the CSC in use, one set per pass
   struct Tiers {
     uint32_t n_med = 0, n_high = 0;
     DevBuf<uint32_t> med, high;
@@ -72,7 +81,7 @@ struct PrPlan {
   DevBuf<uint32_t> hot;
   DevBuf<float> part;
   DevBuf<uint32_t> deg;  // out-degree of each vertex (in the numbering in use)
-  // edge tiles over the CSC in use (instead of the row tiers)
+  // edge tiles over the CSC in use (instead of the row blocks)
   bool tiled = false;
   uint64_t edges = 0;
   uint64_t ntiles = 0;
@@ -163,15 +172,14 @@ __device__ __forceinline__ void finish(uint32_t v, float sum, float base, float 
   contrib[v] = d ? r / (float)d : 0.0f;
 }
 
-// Row v's in-edges swept by pass P: 0 the whole row; in the two-band sweep,
-// 1 the sources below the band boundary (a prefix, rows being sorted) and 2
-// the rest.
+// Row v's in-edges swept by pass P of the two-band sweep: 1 the sources below
+// the band boundary (a prefix, rows being sorted), 2 the rest.
 template <int P>
 __device__ __forceinline__ void row_range(const Csc& g, uint32_t v, uint64_t& s, uint64_t& e) {
   s = g.off[v];
   e = g.off[v + 1];
   if constexpr (P == 1) e = s + g.hot[v];
-  else if constexpr (P == 2) s += g.hot[v];
+  else s += g.hot[v];
 }
 
 // Pass 1 keeps the partial sum; pass 2 adds the rest to it, so every row is
@@ -181,8 +189,7 @@ __device__ __forceinline__ void emit(const Csc& g, uint32_t v, float sum, float 
                                      float* __restrict__ part, float* __restrict__ rank,
                                      float* __restrict__ contrib) {
   if constexpr (P == 1) part[v] = sum;
-  else if constexpr (P == 2) finish(v, part[v] + sum, base, damping, g.deg, rank, contrib);
-  else finish(v, sum, base, damping, g.deg, rank, contrib);
+  else finish(v, part[v] + sum, base, damping, g.deg, rank, contrib);
 }
 
 // Rows with fewer than kMed in-edges in this pass: one lane per row, sources
@@ -512,6 +519,237 @@ __global__ void k_unpermute(const uint32_t* __restrict__ perm, const float* __re
     out[perm[i]] = in[i];
 }
 
+// ---- row blocks ----
+//
+// The CSC's rows are cut into blocks of about kRowEdges in-edges and at most
+// kRowMax rows: row v belongs to block (off[v] + kRowCost * v) / kRowEdges,
+// so the graph alone fixes the blocks.  A workgroup fetches its block's
+// sources with coalesced loads, all its gathers in flight at once, and leaves
+// the contributions in LDS; then a lane sums each short row in order and half
+// a wavefront each longer one (lane-strided, fixed tree), in 64 bits.  Rows of
+// kRowEdges and more (only the last of a block can be one) are cut into
+// chunks, a workgroup each, at the front of the same launch; the workgroup
+// that ends a row's last chunk adds the chunk sums up in a fixed shape.  Ranks
+// are written in the last sweep only, where the caller wants them.
+//
+// Bound by the rate of the gathers: 265 G/s of 4-byte reads at 300 k vertices
+// (4.5 M edges, a sweep of 17 us).  Before, a launch each for rows of one lane
+// / one wavefront / one workgroup and one to end the last spent 46 us there,
+// each waiting for chains of source, contribution, add.  Twenty sweeps, before
+// -> now: 6 k vertices 309 -> 121 us, 300 k 890 -> 366, R-MAT (edge factor 16)
+// s16 429 -> 175, s18 849 -> 324, s20 1907 -> 1435, s21 3371 -> 2941.
+// Blocks of 512 edges: 300 k 427, s20 1659; of 2048: 354, 1424 but 6 k 140,
+// s16 197.  Groups of 8 / 16 lanes: s16 221 / 181; a lane per row below 16 /
+// 64 edges: 300 k 434 / 357, s16 193 / 176.  The 64-bit sums cost nothing
+// that shows.
+
+constexpr uint32_t kRowEdges = 1024;
+constexpr uint32_t kRowCost = 2;
+constexpr uint32_t kRowMax = kRowEdges / kRowCost;
+constexpr uint32_t kRowLane = 32;      // rows below: one lane each
+constexpr uint32_t kRowChunk = 4096;
+constexpr uint32_t kRowGroup = 32;    // longer ones: a group of this many
+constexpr int kRowLoads = kRowEdges / kBlock;           // edges in flight per lane
+
+struct RowView {
+  const uint32_t* row;
+  const uint32_t* row_chunk;
+  const uint32_t* long_row;
+  const uint32_t* chunk_of;
+  const uint64_t* chunk_lo;
+  const uint64_t* chunk_hi;
+  uint32_t* arrived;
+  double* partial;
+  uint32_t n_chunks;
+};
+
+// row[t] = first v with off[v] + kRowCost * v >= t * kRowEdges
+__global__ void k_row_blocks(const uint64_t* __restrict__ off, uint32_t V, uint32_t n, uint32_t* __restrict__ row) {
+  for (uint64_t t = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; t <= n; t += (uint64_t)gridDim.x * blockDim.x) {
+    uint32_t lo = 0, hi = V;
+    while (lo < hi) {
+      const uint32_t mid = lo + (hi - lo) / 2;
+      if (off[mid] + (uint64_t)kRowCost * mid >= t * kRowEdges) hi = mid;
+      else lo = mid + 1;
+    }
+    row[t] = lo;
+  }
+}
+
+__global__ void k_row_long(const uint64_t* __restrict__ off, uint32_t V, uint32_t* __restrict__ list,
+                           uint32_t* __restrict__ n) {
+  for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V; v += (uint64_t)gridDim.x * blockDim.x)
+    if (off[v + 1] - off[v] >= kRowEdges) list[atomicAdd(n, 1u)] = (uint32_t)v;
+}
+
+__global__ void k_row_ranges(const uint64_t* __restrict__ off, const uint32_t* __restrict__ list, uint32_t n,
+                             uint64_t* __restrict__ lo, uint64_t* __restrict__ hi) {
+  for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
+    lo[i] = off[list[i]];
+    hi[i] = off[list[i] + 1];
+  }
+}
+
+// The sum of a row is complete: LAST leaves the rank at the caller's id of
+// the row, the other sweeps leave what the next one gathers.
+template <bool LAST>
+__device__ __forceinline__ void row_done(uint32_t v, double sum, uint32_t deg, float base, float damping,
+                                         const uint32_t* __restrict__ perm, float* __restrict__ out) {
+  const float r = (float)(base + damping * sum);
+  if constexpr (LAST) out[perm ? perm[v] : v] = r;
+  else out[v] = deg ? r / (float)deg : 0.0f;
+}
+
+template <bool LAST>
+__device__ void row_chunk(const Csc& g, const RowView& b, const float* __restrict__ contrib, float base,
+                          float damping, const uint32_t* __restrict__ perm, float* __restrict__ out, double* acc,
+                          uint32_t* flag) {
+  const uint32_t c = blockIdx.x, i = b.chunk_of[c];
+  const uint32_t c0 = b.row_chunk[i], nc = b.row_chunk[i + 1] - c0;
+  const uint64_t lo = b.chunk_lo[c];
+  const uint32_t n = (uint32_t)(b.chunk_hi[c] - lo);  // 1 .. kRowChunk
+  constexpr int kLoads = kRowChunk / kBlock;
+  uint32_t u[kLoads];
+  float x[kLoads];
+#pragma unroll
+  for (int j = 0; j < kLoads; ++j) {
+    const uint32_t k = j * kBlock + threadIdx.x;
+    u[j] = ld_src(g.src + lo + (k < n ? k : n - 1));
+  }
+#pragma unroll
+  for (int j = 0; j < kLoads; ++j) x[j] = contrib[u[j]];
+  double sum = 0.0;
+#pragma unroll
+  for (int j = 0; j < kLoads; ++j) sum += j * kBlock + threadIdx.x < n ? x[j] : 0.0f;
+  auto reduce = [&](double s) {
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) s += __shfl_xor(s, d, 64);
+    if (__lane_id() == 0) acc[threadIdx.x / 64] = s;
+    __syncthreads();
+    s = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+    __syncthreads();
+    return s;
+  };
+  sum = reduce(sum);
+  if (nc > 1) {
+    if (threadIdx.x == 0) {
+      __hip_atomic_store(&b.partial[c], sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const uint32_t done = __hip_atomic_fetch_add(&b.arrived[i], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+      *flag = done + 1 == nc;
+      // the next sweep counts from zero again
+      if (done + 1 == nc) __hip_atomic_store(&b.arrived[i], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (!*flag) return;  // uniform
+    sum = 0.0;
+    for (uint32_t k = threadIdx.x; k < nc; k += kBlock)
+      sum += __hip_atomic_load(&b.partial[c0 + k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    sum = reduce(sum);
+  }
+  if (threadIdx.x == 0) {
+    const uint32_t v = b.long_row[i];
+    row_done<LAST>(v, sum, LAST ? 0u : g.deg[v], base, damping, perm, out);
+  }
+}
+
+template <bool LAST>
+__global__ __launch_bounds__(kBlock) void k_pr_rows(Csc g, RowView b, const float* __restrict__ contrib, float base,
+                                                    float damping, const uint32_t* __restrict__ perm,
+                                                    float* __restrict__ out) {
+  __shared__ float val[2 * kRowEdges + 4];
+  __shared__ double total[kRowMax];
+  __shared__ uint32_t big[2 * kRowEdges / kRowLane];
+  __shared__ uint32_t n_big;
+  if (blockIdx.x < b.n_chunks) {
+    row_chunk<LAST>(g, b, contrib, base, damping, perm, out, total, &n_big);
+    return;
+  }
+  const uint32_t t = blockIdx.x - b.n_chunks;
+  const uint32_t r0 = b.row[t];
+  uint32_t rows = b.row[t + 1] - r0;
+  if (!rows) return;  // inside a long row
+  const uint64_t e0 = g.off[r0];
+  uint32_t n;  // edges of the block's short rows, below 2 * kRowEdges
+  {
+    const uint64_t a = g.off[r0 + rows - 1], z = g.off[r0 + rows];
+    if (z - a >= kRowEdges) --rows, n = (uint32_t)(a - e0);
+    else n = (uint32_t)(z - e0);
+  }
+  constexpr int kOwn = kRowMax / kBlock;
+  uint32_t s[kOwn], d[kOwn], deg[kOwn];
+#pragma unroll
+  for (int q = 0; q < kOwn; ++q) {
+    const uint32_t i = q * kBlock + threadIdx.x;
+    s[q] = d[q] = deg[q] = 0;
+    if (i < rows) {
+      const uint64_t x = g.off[r0 + i];
+      s[q] = (uint32_t)(x - e0);
+      d[q] = (uint32_t)(g.off[r0 + i + 1] - x);
+      if constexpr (!LAST) deg[q] = g.deg[r0 + i];
+    }
+  }
+  if (threadIdx.x == 0) n_big = 0;
+  for (uint32_t k0 = 0; k0 < n; k0 += kRowLoads * kBlock) {
+    uint32_t u[kRowLoads];
+    float x[kRowLoads];
+#pragma unroll
+    for (int j = 0; j < kRowLoads; ++j) {
+      const uint32_t k = k0 + j * kBlock + threadIdx.x;
+      u[j] = ld_src(g.src + e0 + (k < n ? k : n - 1));
+    }
+#pragma unroll
+    for (int j = 0; j < kRowLoads; ++j) x[j] = contrib[u[j]];
+#pragma unroll
+    for (int j = 0; j < kRowLoads; ++j) {
+      const uint32_t k = k0 + j * kBlock + threadIdx.x;
+      if (k < n) val[k] = x[j];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < kOwn; ++q) {
+    const uint32_t i = q * kBlock + threadIdx.x;
+    if (d[q] < kRowLane) {
+      double sum = 0.0;
+      for (uint32_t k = 0; k < d[q]; k += 4) {
+        float x[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[j] = val[s[q] + k + j];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sum += k + j < d[q] ? x[j] : 0.0f;
+      }
+      if (i < rows) row_done<LAST>(r0 + i, sum, deg[q], base, damping, perm, out);
+    } else {
+      big[atomicAdd(&n_big, 1u)] = s[q] | d[q] << 12 | i << 23;
+    }
+  }
+  __syncthreads();
+  const uint32_t nb = n_big;
+  if (!nb) return;
+  const uint32_t lane = threadIdx.x % kRowGroup;
+  for (uint32_t w = threadIdx.x / kRowGroup; w < nb; w += kBlock / kRowGroup) {
+    const uint32_t e = big[w], start = e & 4095, len = e >> 12 & 2047;
+    double sum = 0.0;
+    for (uint32_t k = lane; k < len; k += 4 * kRowGroup) {
+      float x[4];
+#pragma unroll
+      for (uint32_t j = 0; j < 4; ++j) x[j] = val[k + j * kRowGroup < len ? start + k + j * kRowGroup : start];
+#pragma unroll
+      for (uint32_t j = 0; j < 4; ++j) sum += k + j * kRowGroup < len ? x[j] : 0.0f;
+    }
+#pragma unroll
+    for (int h = kRowGroup / 2; h >= 1; h >>= 1) sum += __shfl_xor(sum, h, kRowGroup);
+    if (lane == 0) total[e >> 23] = sum;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < kOwn; ++q) {
+    const uint32_t i = q * kBlock + threadIdx.x;
+    if (d[q] >= kRowLane) row_done<LAST>(r0 + i, total[i], deg[q], base, damping, perm, out);
+  }
+}
+static_assert(2 * kRowEdges <= 1u << 12 && kRowMax <= 1u << 9 && kBlock == 256, "packed row of a block");
+
 // ---- segmented layout construction ----
 
 // key = window(u) << 2b | v << b | u for edge u -> v
@@ -680,6 +918,59 @@ int build_tiers(const Csc& g, PrPlan::Tiers& t, hipStream_t s) {
     CG_HIP(hipMemcpyAsync(t.chunk_hi.p, chi.data(), chi.size() * 8, hipMemcpyHostToDevice, s));
   }
   CG_HIP(hipMemcpyAsync(t.row_chunk.p, first.data(), first.size() * 4, hipMemcpyHostToDevice, s));
+  CG_HIP(hipStreamSynchronize(s));
+  return CG_OK;
+}
+
+// Row blocks and the chunks of the long rows over a CSC.
+int build_rows(const uint64_t* off, uint32_t V, uint64_t E, PrPlan::RowBlocks& b, hipStream_t s) {
+  b.n = (uint32_t)((E + (uint64_t)kRowCost * V + kRowEdges - 1) / kRowEdges);
+  CG_TRY(b.row.ensure(b.n + 1));
+  const uint64_t max_long = E / kRowEdges;
+  DevBuf<uint32_t> cnt;
+  CG_TRY(cnt.ensure(1));
+  CG_TRY(b.long_row.ensure(max_long ? max_long : 1));
+  CG_HIP(hipMemsetAsync(cnt.p, 0, sizeof(uint32_t), s));
+  hipLaunchKernelGGL(k_row_blocks, dim3(grid_of(b.n + 1)), dim3(kBlock), 0, s, off, V, b.n, b.row.p);
+  PR_LAUNCH_OK();
+  hipLaunchKernelGGL(k_row_long, dim3(grid_of(V)), dim3(kBlock), 0, s, off, V, b.long_row.p, cnt.p);
+  PR_LAUNCH_OK();
+  uint32_t n = 0;
+  CG_HIP(hipMemcpyAsync(&n, cnt.p, sizeof(n), hipMemcpyDeviceToHost, s));
+  CG_HIP(hipStreamSynchronize(s));
+  if (!n) return CG_OK;
+  DevBuf<uint64_t> lo, hi;
+  CG_TRY(lo.ensure(n));
+  CG_TRY(hi.ensure(n));
+  hipLaunchKernelGGL(k_row_ranges, dim3(grid_of(n)), dim3(kBlock), 0, s, off, b.long_row.p, n, lo.p, hi.p);
+  PR_LAUNCH_OK();
+  std::vector<uint64_t> hl(n), hh(n);
+  CG_HIP(hipMemcpyAsync(hl.data(), lo.p, n * 8ull, hipMemcpyDeviceToHost, s));
+  CG_HIP(hipMemcpyAsync(hh.data(), hi.p, n * 8ull, hipMemcpyDeviceToHost, s));
+  CG_HIP(hipStreamSynchronize(s));
+  std::vector<uint64_t> clo, chi;
+  std::vector<uint32_t> of, first(n + 1);
+  for (uint32_t i = 0; i < n; ++i) {
+    first[i] = (uint32_t)clo.size();
+    for (uint64_t a = hl[i]; a < hh[i]; a += kRowChunk) {
+      clo.push_back(a);
+      chi.push_back(std::min<uint64_t>(a + kRowChunk, hh[i]));
+      of.push_back(i);
+    }
+  }
+  first[n] = (uint32_t)clo.size();
+  b.n_chunks = (uint32_t)clo.size();
+  CG_TRY(b.chunk_lo.ensure(clo.size()));
+  CG_TRY(b.chunk_hi.ensure(chi.size()));
+  CG_TRY(b.chunk_of.ensure(of.size()));
+  CG_TRY(b.row_chunk.ensure(first.size()));
+  CG_TRY(b.partial.ensure(clo.size()));
+  CG_TRY(b.arrived.ensure(n));
+  CG_HIP(hipMemcpyAsync(b.chunk_lo.p, clo.data(), clo.size() * 8, hipMemcpyHostToDevice, s));
+  CG_HIP(hipMemcpyAsync(b.chunk_hi.p, chi.data(), chi.size() * 8, hipMemcpyHostToDevice, s));
+  CG_HIP(hipMemcpyAsync(b.chunk_of.p, of.data(), of.size() * 4, hipMemcpyHostToDevice, s));
+  CG_HIP(hipMemcpyAsync(b.row_chunk.p, first.data(), first.size() * 4, hipMemcpyHostToDevice, s));
+  CG_HIP(hipMemsetAsync(b.arrived.p, 0, n * sizeof(uint32_t), s));
   CG_HIP(hipStreamSynchronize(s));
   return CG_OK;
 }
@@ -1697,7 +1988,6 @@ int pr_plan_create(cg_graph* graph, uint32_t layout, uint32_t seg_log2, uint32_t
     st = build_relabelled(graph, p, s);
   } else {
     st = build_degrees(g, p, s);
-    if (st == CG_OK) st = build_tiers<0>(Csc{g.in_off, g.in_src, p->deg.p, g.V, nullptr}, p->tiers[0], s);
     p->layout = kLayoutPlain;
   }
   if (st == CG_OK && p->layout == kLayoutRelabel) {
@@ -1706,10 +1996,11 @@ int pr_plan_create(cg_graph* graph, uint32_t layout, uint32_t seg_log2, uint32_t
     } else if (kernel == 2) {
       st = build_tiles(p->r_off.p, g.V, E, p, s);
     } else {
-      st = build_tiers<0>(Csc{p->r_off.p, p->r_src.p, p->deg.p, g.V, nullptr}, p->tiers[0], s);
+      st = build_rows(p->r_off.p, g.V, E, p->rows, s);
     }
-  } else if (st == CG_OK && p->layout == kLayoutPlain && kernel == 2) {
-    st = build_tiles(g.in_off, g.V, E, p, s);
+  } else if (st == CG_OK && p->layout == kLayoutPlain) {
+    if (kernel == 2) st = build_tiles(g.in_off, g.V, E, p, s);
+    else st = build_rows(g.in_off, g.V, E, p->rows, s);
   }
   if (st != CG_OK) {
     delete p;
@@ -1737,12 +2028,16 @@ int pr_run(const DevGraph& g, PrPlan* plan, int iters, float damping, float* ran
   const Csc csc = relabel ? Csc{plan->r_off.p, plan->r_src.p, plan->deg.p, V, plan->hot.p}
                           : Csc{g.in_off, g.in_src, plan->deg.p, V, nullptr};
   const uint64_t plan_edges = plan->edges;
-  hipLaunchKernelGGL(k_pr_init, dim3(std::min<unsigned>(vblocks, 65536)), dim3(kBlock), 0, s, V, plan->deg.p,
-                     1.0f / (float)V, rank, contrib);
-  float* r_cur = rank;
-  float* r_nxt = tmp_rank;
+  // the ranks alternate between two buffers and end in the caller's; the row
+  // blocks write them there in the last sweep only
+  const bool rows = plan->rows.n != 0;
+  const bool swapped = !rows && (iters + (relabel ? 1 : 0)) % 2;
+  float* r_cur = swapped ? tmp_rank : rank;
+  float* r_nxt = swapped ? rank : tmp_rank;
   float* c_cur = contrib;
   float* c_nxt = contrib2;
+  hipLaunchKernelGGL(k_pr_init, dim3(std::min<unsigned>(vblocks, 65536)), dim3(kBlock), 0, s, V, plan->deg.p,
+                     1.0f / (float)V, r_cur, contrib);
   hipEvent_t a = nullptr, b = nullptr;
   if (profile) {
     CG_HIP(hipEventCreate(&a));
@@ -1807,7 +2102,15 @@ int pr_run(const DevGraph& g, PrPlan* plan, int iters, float damping, float* ran
       launch_tiers<1>(csc, plan->tiers[0], vblocks, c_cur, base, damping, plan->part.p, r_nxt, c_nxt, s);
       launch_tiers<2>(csc, plan->tiers[1], vblocks, c_cur, base, damping, plan->part.p, r_nxt, c_nxt, s);
     } else {
-      launch_tiers<0>(csc, plan->tiers[0], vblocks, c_cur, base, damping, nullptr, r_nxt, c_nxt, s);
+      const PrPlan::RowBlocks& b = plan->rows;
+      const RowView view{b.row.p,      b.row_chunk.p, b.long_row.p, b.chunk_of.p, b.chunk_lo.p,
+                         b.chunk_hi.p, b.arrived.p,   b.partial.p,  b.n_chunks};
+      if (it + 1 < iters)
+        hipLaunchKernelGGL(k_pr_rows<false>, dim3(b.n_chunks + b.n), dim3(kBlock), 0, s, csc, view, c_cur, base,
+                           damping, nullptr, c_nxt);
+      else
+        hipLaunchKernelGGL(k_pr_rows<true>, dim3(b.n_chunks + b.n), dim3(kBlock), 0, s, csc, view, c_cur, base,
+                           damping, relabel ? plan->perm.p : nullptr, rank);
     }
     if (profile) {
       CG_HIP(hipEventRecord(b, s));
@@ -1819,15 +2122,13 @@ int pr_run(const DevGraph& g, PrPlan* plan, int iters, float damping, float* ran
     std::swap(r_cur, r_nxt);
     std::swap(c_cur, c_nxt);
   }
-  if (relabel) {
-    // back to the caller's ids: r_nxt is free after the last swap
+  if (relabel && !rows) {
+    // back to the caller's ids: r_nxt is the caller's buffer after the last swap
     hipLaunchKernelGGL(k_unpermute, dim3(std::min<unsigned>(vblocks, 65536)), dim3(kBlock), 0, s, plan->perm.p,
                        r_cur, V, r_nxt);
-    std::swap(r_cur, r_nxt);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return set_error(CG_ERR_HIP, "PageRank kernels: %s", hipGetErrorString(e));
-  if (r_cur != rank) CG_HIP(hipMemcpyAsync(rank, r_cur, (uint64_t)V * sizeof(float), hipMemcpyDeviceToDevice, s));
   CG_HIP(hipStreamSynchronize(s));
   if (profile) {
     (void)hipEventDestroy(a);

@@ -1,0 +1,47 @@
+"""PageRank over blocks of consecutive rows (csrc/pagerank.hip): rows around
+the lane / wavefront / chunk limits, blocks of empty rows, ranks written in the
+caller's ids by the last sweep.  FP64 oracle; the bound is FP32's rounding
+(2^-24 of the total mass per addition along the longest chain, 31 + 6 adds in a
+block, 16 + 8 per chunk, over 20 damped iterations: 1e-6 of the mass of 1 with
+slack), and run-to-run bit-identity."""
+import numpy as np
+import pytest
+
+import cggraph_amd as cg
+
+pytestmark = pytest.mark.gpu
+
+PR = 3
+
+
+def graphs(oracle):
+    rng = np.random.default_rng(3)
+    deg = [31, 32, 33, 63, 64, 65, 2047, 2048, 2049, 4095, 4096, 4097, 8192, 20481, 1, 0, 2047, 2047, 31, 31]
+    V = 4000  # the rows above, then empty ones (more than a block of them), then a few with one edge
+    dst = np.concatenate([np.repeat(np.arange(len(deg)), deg), np.arange(V - 100, V)])
+    src = rng.integers(0, V, len(dst))
+    yield "limits", oracle.csr_build(V, src.astype(np.uint32), dst.astype(np.uint32))
+    # the last row of a block takes it to just below twice the block's edges
+    deg = np.full(70, 30)
+    deg[67:] = 2047
+    dst = np.repeat(np.arange(70), deg)
+    yield "full block", oracle.csr_build(70, rng.integers(0, 70, len(dst)).astype(np.uint32), dst.astype(np.uint32))
+    yield "one edge", oracle.csr_build(2, np.array([1], np.uint32), np.array([0], np.uint32))
+    yield "no edge", oracle.csr_build(513, np.zeros(0, np.uint32), np.zeros(0, np.uint32))
+    yield "renumbered", oracle.rmat_graph(17, 9, seed=6, weights=None)
+
+
+@pytest.mark.parametrize("layout", [1, 2])
+def test_row_blocks(oracle, layout):
+    for name, og in graphs(oracle):
+        g = cg.Graph.from_csr(og.offsets, og.dest)
+        for iters in (0, 1, 2, 20):
+            e = cg.Engine(g, PR, pr_layout=layout, pr_iterations=iters)
+            r1, _ = e.run()
+            r2, _ = e.run()
+            e.close()
+            assert np.array_equal(r1.view(np.uint32), r2.view(np.uint32)), (name, iters)
+            ref = oracle.pagerank64(og, iters, 0.85)
+            l1 = float(np.abs(r1.astype(np.float64) - ref).sum())
+            assert l1 <= 1e-6, (name, iters, l1)
+        g.close()
