@@ -309,8 +309,8 @@ int cg_options_default(cg_options* o) {
   o->heavy_active_vertices = 16384;
   o->heavy_active_edges = 25000000ull;
   o->bin_wave = 32;
-  o->bin_chunk = 4096;
-  o->chunk_edges = 2048;
+  o->bin_chunk = kBinChunk;
+  o->chunk_edges = kChunkEdges;
   o->sched_mode = CG_SCHED_GPU;
   o->forced_choice = 0;
   o->cpu_threads = 0;
@@ -655,7 +655,7 @@ int cg_engine_create(const cg_graph* cg, int algorithm, int engine_type, int use
     CG_TRY(e->bm[1].ensure(words));
     CG_TRY(e->q_small.ensure(V));
     CG_TRY(e->q_med.ensure(V));
-    uint32_t min_chunk = e->opt.chunk_edges;
+    uint32_t min_chunk = std::min(e->opt.chunk_edges, chunk_edges_for(g->E));
     // narrow frontiers on the GPU schedule run in a level cluster; traces,
     // profiles and bottom-up min steps are the per-iteration pipeline's
     const bool cluster = e->opt.sched_mode == CG_SCHED_GPU && !e->partial && !e->opt.trace_path && !e->opt.profile &&

@@ -591,7 +591,20 @@ int engine_run(cg_engine* e, uint32_t root, cg_run_stats* rs) {
     choice_tiers.wave[k] = k ? kTierSets[k].bin_wave : e->opt.bin_wave;
     choice_tiers.chunk[k] = k ? kTierSets[k].bin_chunk : e->opt.bin_chunk;
   }
-  const Bins fbins{e->opt.bin_wave, e->opt.bin_chunk, e->opt.chunk_edges, e->opt.expand_grid};
+  Bins fbins{e->opt.bin_wave, e->opt.bin_chunk, e->opt.chunk_edges, e->opt.expand_grid};
+  if (mode == CG_SCHED_GPU && fbins.bin_chunk == kBinChunk && fbins.chunk_edges == kChunkEdges) {
+    // the default tiers, by the graph's size (chunk_edges_for)
+    fbins.chunk_edges = chunk_edges_for(g.E);
+    fbins.bin_chunk = std::max(fbins.bin_wave, 2 * fbins.chunk_edges);
+  }
+  // SSSP's first frontier is the root alone, whose edges go to as many
+  // wavefronts as a BFS frontier's do (kChunkSpread): 37 k edges 55 -> ~5 us
+  Bins root_bins = fbins;
+  if (mode == CG_SCHED_GPU && alg == CG_SSSP) {
+    uint32_t& ce = root_bins.chunk_edges;
+    while (ce > (uint32_t)kWave && e->caller_g->max_outdeg < (uint64_t)ce * kChunkSpread) ce >>= 1;
+    root_bins.bin_chunk = std::min(root_bins.bin_chunk, 2 * ce);
+  }
   // Pure GPU schedule: iteration it + 1 is queued before the host reads the
   // statistics of iteration it, so the host's launch work overlaps the GPU.
   // The iteration after the last one finds an empty frontier and does nothing;
@@ -689,11 +702,12 @@ int engine_run(cg_engine* e, uint32_t root, cg_run_stats* rs) {
     const int sl = k & 1, c = (k - 1) & 1;
     DevStats* dk = e->st.p + sl;
     if (fused) {
-      Bins xb = fbins;
+      const Bins& cb = k == 1 ? root_bins : fbins;
+      Bins xb = cb;
       if (last_m < kTailEdges && last_m <= prev_m && (xb.grid_cap == 0 || xb.grid_cap > kTailGrid))
         xb.grid_cap = kTailGrid;
       uint32_t nparts = 0;
-      CG_TRY(launch_compact_fused(e->bm[c].p, e->bm[c ^ 1].p, words, dg, fbins, e->q_small.p, e->q_med.p,
+      CG_TRY(launch_compact_fused(e->bm[c].p, e->bm[c ^ 1].p, words, dg, cb, e->q_small.p, e->q_med.p,
                                   e->q_chunk.p, dk, e->val.p, hub, e->parts.p, &nparts, e->run_state.p, s,
                                   early_learned ? &choice_tiers : nullptr));
       const int tp = k & 3;

@@ -38,6 +38,21 @@ static_assert(sizeof(DevStats) % 8 == 0, "DevStats layout");
 // one wavefront's width), so that a lone hub spreads over the machine; at
 // most 2 * kChunkSpread extra items come of it.
 constexpr uint32_t kChunkSpread = 2048;
+// The default push tiers, and what they become on a graph of E edges under
+// the GPU schedule: the expansion's 8192 wavefronts share a frontier's edges,
+// and one that takes a 4096-edge vertex or a 2048-edge chunk where an even
+// share is 1400 edges ends long after the others.  A chunk is an eighth of an
+// even share of all edges, 256 at least, and a vertex of two chunks is split
+// (SSSP, 4096 / 2048 -> the rule's: 1 M vertices and 12 M edges 1128 -> 945 us,
+// 200 k / 2.3 M 839 -> 645, R-MAT s20 1523 -> 1299, s22 1942 -> 1809; chunks of
+// 128: 977, 640, 1316, 2075; of 256 at s23 4962 against 4794 of the rule's
+// 1024.  BFS: s14 114 -> 70, s15 104 -> 62, s19 140 -> 135, s22 245 -> 238).
+constexpr uint32_t kBinChunk = 4096, kChunkEdges = 2048;
+inline uint32_t chunk_edges_for(uint64_t E) {
+  uint32_t ce = kChunkEdges;
+  while (ce > 256 && E < (uint64_t)ce * 8 * 8192) ce >>= 1;
+  return ce;
+}
 
 // Counters written by many wavefronts are striped over kStripes cache lines
 // so that their atomics do not serialise on one address.

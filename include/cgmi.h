@@ -97,7 +97,9 @@ typedef struct cg_options {
   uint64_t heavy_active_edges;    /* HEAVY_ACTIVE_EDGES 25 000 000 (CGgraph_engine.cuh:22) */
   uint32_t bin_wave;              /* degree >= bin_wave: one wavefront per vertex */
   uint32_t bin_chunk;             /* degree >= bin_chunk: split into edge chunks */
-  uint32_t chunk_edges;           /* edges per chunk of a split vertex */
+  uint32_t chunk_edges;           /* edges per chunk of a split vertex; the default pair
+                                     (bin_chunk 4096, chunk_edges 2048) shrinks with the
+                                     graph under the GPU schedule, to 512 and 256 */
   int sched_mode;                 /* CG_SCHED_* */
   int forced_choice;              /* 0..CG_NUM_CHOICES-1 for CG_SCHED_FORCED */
   int cpu_threads;                /* host team size; 0 = all cores */
