@@ -685,7 +685,7 @@ int cg_engine_create(const cg_graph* cg, int algorithm, int engine_type, int use
     e->hst_map_dev = e->hst_map.device_ptr();
     if (!e->hst_map_dev) return set_error(CG_ERR_HIP, "mapped statistics buffer has no device address");
     CG_TRY(e->acc.ensure(kAccSlots));
-    CG_TRY(e->parts.ensure(stats_parts_needed(words)));
+    CG_TRY(e->parts.ensure(fused_parts_needed(words)));
     CG_TRY(e->stripes.ensure(kStripeWords));
     CG_TRY(e->run_state.ensure(2));
     if (algorithm == CG_BFS) CG_TRY(e->bfs_cnt.ensure(2 * kBfsCntWords));

@@ -27,6 +27,7 @@
 // kLongRow edges go to a list that a second kernel takes a workgroup each, so
 // that no hub outside z's reach holds one wavefront up.
 #include "kernels.hpp"
+#include "wave.hpp"
 
 namespace cg {
 
@@ -38,18 +39,6 @@ constexpr uint32_t kLaneEdges = 32;
 constexpr uint64_t kLongRow = 16384;
 
 __device__ __forceinline__ uint32_t min_u32(uint32_t a, uint32_t b) { return a < b ? a : b; }
-
-__device__ __forceinline__ uint32_t wave_min(uint32_t x) {
-#pragma unroll
-  for (int d = kWave / 2; d >= 1; d >>= 1) x = min_u32(x, __shfl_xor(x, d, kWave));
-  return x;
-}
-
-__device__ __forceinline__ unsigned long long wave_sum(unsigned long long x) {
-#pragma unroll
-  for (int d = kWave / 2; d >= 1; d >>= 1) x += __shfl_xor(x, d, kWave);
-  return x;
-}
 
 // Whether round r has anything to do: the first always, the second if the
 // vertices changed in the one before send many edges.  Every workgroup takes
@@ -108,7 +97,7 @@ __global__ __launch_bounds__(kBlock) void k_cc_pull(DevGraph g, uint64_t E, uint
         x = min_u32(x, min_u32(min_u32(u[0], u[1]), min_u32(u[2], u[3])));
         if (__ballot(x == z)) break;
       }
-      x = wave_min(x);
+      x = wave_min_u32(x);
       if ((int)lane == l) best = min_u32(best, x);
     }
     const bool fell = best < cur;
@@ -119,7 +108,7 @@ __global__ __launch_bounds__(kBlock) void k_cc_pull(DevGraph g, uint64_t E, uint
     const uint64_t mask = __ballot(fell);
     if (lane == 0) changed_bm[wd] = mask;
   }
-  m = wave_sum(m);
+  m = wave_sum_u64(m);
   if (lane == 0 && m) atomicAdd(&cnt[r].edges[(blockIdx.x % kStripes) * kCcStride], m);
 }
 
@@ -145,7 +134,7 @@ __global__ __launch_bounds__(kLongBlock) void k_cc_pull_long(DevGraph g, uint64_
       x = min_u32(x, min_u32(min_u32(u[0], u[1]), min_u32(u[2], u[3])));
       if (x == z) break;
     }
-    x = wave_min(x);
+    x = wave_min_u32(x);
     if (__lane_id() == 0) atomicMin(&best, x);
     __syncthreads();
     if (threadIdx.x == 0 && best < val[v]) {
@@ -164,7 +153,7 @@ __global__ __launch_bounds__(kBlock) void k_first_source(const uint32_t* __restr
   for (uint64_t v = blockIdx.x * (uint64_t)kBlock + threadIdx.x; v < V && x == 0xFFFFFFFFu;
        v += (uint64_t)gridDim.x * kBlock)
     if (deg[v]) x = (uint32_t)v;
-  x = wave_min(x);
+  x = wave_min_u32(x);
   if (__lane_id() == 0 && x != 0xFFFFFFFFu) atomicMin(out, x);
 }
 
@@ -176,7 +165,7 @@ __global__ __launch_bounds__(kBlock) void k_source_reach(DevGraph g, const uint3
   unsigned long long x = 0;
   for (uint64_t k = s + blockIdx.x * (uint64_t)kBlock + threadIdx.x; k < e; k += (uint64_t)gridDim.x * kBlock)
     x += g.deg[g.dst[k]];
-  x = wave_sum(x);
+  x = wave_sum_u64(x);
   if (__lane_id() == 0 && x) atomicAdd(m, x);
 }
 

@@ -1,6 +1,8 @@
 // The level cluster of cluster.hpp: device code and launcher.
 #include "cluster.hpp"
 
+#include "wave.hpp"
+
 namespace cg {
 
 namespace {
@@ -20,22 +22,6 @@ template <class T>
 __device__ __forceinline__ T add_agent(T* p, T x) {
   return __hip_atomic_fetch_add(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-
-// Inclusive prefix sum over the wavefront in six DPP adds: a shuffle goes
-// through LDS (about 60 cycles each, dependent), which a level cannot hide.
-__device__ __forceinline__ uint32_t wave_scan(uint32_t x) {
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false);  // row_shr:1
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false);  // row_shr:2
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false);  // row_shr:4
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false);  // row_shr:8
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);  // row_bcast:15 to rows 1, 3
-  x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);  // row_bcast:31 to rows 2, 3
-  return x;
-}
-__device__ __forceinline__ uint32_t lane_value(uint32_t x, uint32_t l) {  // l wave-uniform
-  return (uint32_t)__builtin_amdgcn_readlane((int)x, (int)l);
-}
-__device__ __forceinline__ uint32_t wave_sum(uint32_t x) { return lane_value(wave_scan(x), kWave - 1); }
 
 constexpr unsigned long long kMask40 = (1ull << 40) - 1;
 // A level's report, the sum of its workgroups': arrivals (6 bits) | those that
@@ -113,7 +99,7 @@ __device__ __forceinline__ void cluster_run(ClusterShared& S, const ClusterJob& 
   // counts to the level's report and waits until all have.  The queue read in
   // this level becomes the next one to fill.
   auto barrier = [&](uint32_t lvl, uint32_t qp) {
-    const uint32_t ms = wave_sum(m);
+    const uint32_t ms = wave_sum_u32(m);
     const bool any_stop = __ballot(stop != 0) != 0;
     if (lane == 0) {
       if (nv) {
@@ -325,13 +311,13 @@ __device__ __forceinline__ void cluster_run(ClusterShared& S, const ClusterJob& 
     if constexpr (ALG == CG_BFS) {
       // the step that made the frontier counted it
       if (t < (uint32_t)kStripes) c = (uint32_t)J.bfs_cnt[(size_t)((k - 1) & 1) * kBfsCntWords + t * kBfsCntStride];
-      c = wave_sum(c < kShareMax ? c : kShareMax);
+      c = wave_sum_u32(c < kShareMax ? c : kShareMax);
       if (wv == 0 && id == 0) nv = c;
     } else {
       for (uint64_t i = gt; i < J.words; i += nthreads) {
         c += (uint32_t)__popcll(in[i]);
       }
-      nv = wave_sum(c);
+      nv = wave_sum_u32(c);
     }
     barrier(L++, 0);
     const uint32_t total = S.view.n;
@@ -581,8 +567,8 @@ __device__ __forceinline__ void cluster_run(ClusterShared& S, const ClusterJob& 
   // ---- the end ----
   const LevelView V = S.view;
   if constexpr (ALG != CG_BFS) {
-    const unsigned long long es = ((unsigned long long)wave_sum(e_done >> 16) << 16) + wave_sum(e_done & 0xFFFFu);
-    v_done = wave_sum(v_done);
+    const unsigned long long es = ((unsigned long long)wave_sum_u32(e_done >> 16) << 16) + wave_sum_u32(e_done & 0xFFFFu);
+    v_done = wave_sum_u32(v_done);
     if (lane == 0 && v_done) {
       (void)add_agent(&ctl->edges_done, es);
       (void)add_agent(&ctl->verts_done, (unsigned long long)v_done);

@@ -144,6 +144,7 @@ int launch_init_run_state(RunState* rs, uint64_t visited, hipStream_t s);
 // decision on the device (the rule of the host's beamer_pull, state in rs) and
 // leaves it in st->choice (1 bottom-up, 0 push), for the kernels queued behind.
 uint64_t stats_parts_needed(uint64_t words);
+uint64_t fused_parts_needed(uint64_t words);  // what launch_compact_fused writes too
 // prev not NULL: the other statistics slot, whose deferral counts (left by the
 // previous iteration's compaction) are published as n_def_prev / m_def_prev.
 int launch_stats(const uint64_t* in, uint64_t* zero_me, uint64_t words, const DevGraph& g,
@@ -182,7 +183,7 @@ int launch_compact(const uint64_t* in, uint64_t words, const DevGraph& g, const 
 // (lengths into st, whose counters start at zero), every word of `out` (zero,
 // or the hubs kept waiting under `hub`) and one statistics partial per
 // workgroup into `parts` (*nparts set by the launcher, at most
-// stats_parts_needed(words) - 1).  The hub threshold is st->min_val +
+// fused_parts_needed(words) - 1).  The hub threshold is st->min_val +
 // hub.delta.  With g.deg and g.xval, a frontier vertex whose value is the
 // one its out-edges were last relaxed with is dropped: its bit is cleared in
 // `in`, and it is neither queued nor counted.  launch_fused_finish reduces

@@ -25,9 +25,12 @@
 #include <chrono>
 #include <cstddef>
 
+#include <algorithm>
+
 #include "kernels.hpp"
 #include "mlp_dev.hpp"
 #include "sched.hpp"
+#include "wave.hpp"
 
 namespace cg {
 
@@ -41,31 +44,6 @@ constexpr int kFinishParts = 4;
 
 __device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
 __device__ __forceinline__ uint32_t wave_id() { return threadIdx.x / kWave; }
-
-// Exclusive prefix sum over the 64 lanes; every lane must be active.
-__device__ __forceinline__ uint32_t wave_excl_scan(uint32_t x, uint32_t* total) {
-  const uint32_t lane = lane_id();
-  uint32_t v = x;
-#pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    uint32_t t = __shfl_up(v, d, kWave);
-    if (lane >= (uint32_t)d) v += t;
-  }
-  *total = __shfl(v, kWave - 1, kWave);
-  return v - x;
-}
-
-__device__ __forceinline__ uint64_t wave_sum_u64(uint64_t x) {
-#pragma unroll
-  for (int d = kWave / 2; d >= 1; d >>= 1) x += __shfl_xor(x, d, kWave);
-  return x;
-}
-
-__device__ __forceinline__ uint32_t wave_sum_u32(uint32_t x) {
-#pragma unroll
-  for (int d = kWave / 2; d >= 1; d >>= 1) x += __shfl_xor(x, d, kWave);
-  return x;
-}
 
 __device__ __forceinline__ uint32_t hist_bin(uint64_t deg) {
   uint32_t l = 63 - __clzll(deg + 1);  // floor(log2(deg + 1))
@@ -98,15 +76,6 @@ __device__ __forceinline__ void stripe_add(uint32_t* stripes, uint32_t v) {
 __device__ __forceinline__ void stripe_min(uint32_t* stripes, uint32_t v) {
   if (v != 0xFFFFFFFFu && lane_id() == 0)
     atomicMin(stripes + kStripeMinBase + (blockIdx.x % kStripes) * kStripeStride, v);
-}
-
-__device__ __forceinline__ uint32_t wave_min_u32(uint32_t x) {
-#pragma unroll
-  for (int d = kWave / 2; d >= 1; d >>= 1) {
-    const uint32_t o = __shfl_xor(x, d, kWave);
-    x = o < x ? o : x;
-  }
-  return x;
 }
 
 enum { ALG_BFS = CG_BFS, ALG_SSSP = CG_SSSP, ALG_CC = CG_CC };
@@ -518,6 +487,28 @@ __device__ __forceinline__ void stats_block_part(const StatsPart& p, StatsPart* 
   }
 }
 
+// The same over a workgroup of NB threads, whose wavefronts' partials the
+// lanes of the first one add up.
+template <int NB>
+__device__ __forceinline__ void stats_wide_part(const StatsPart& p, StatsPart* __restrict__ parts) {
+  constexpr uint32_t kWaves = NB / kWave;
+  __shared__ StatsPart wpart[kWaves];
+  if (lane_id() == 0) wpart[wave_id()] = p;
+  __syncthreads();
+  if (threadIdx.x >= kWave) return;
+  StatsPart b{};
+  if (lane_id() < kWaves) b = wpart[lane_id()];
+  b.n_active = wave_sum_u32(b.n_active);
+  b.n_zero = wave_sum_u32(b.n_zero);
+  b.m_active = wave_sum_u64(b.m_active);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) b.hist[k] = wave_sum_u32(b.hist[k]);
+  b.n_def = wave_sum_u32(b.n_def);
+  b.m_def = wave_sum_u64(b.m_def);
+  b.min_val = 0xFFFFFFFFu;
+  if (lane_id() == 0) parts[blockIdx.x] = b;
+}
+
 // One workgroup: fixed-order reduction of the partials, first-visit stripes,
 // run state, features and (with weights) the scheduler network, then the
 // counters of the next compaction and the publication to mapped host memory
@@ -884,12 +875,8 @@ __global__ __launch_bounds__(kBlock) void k_compact(const uint64_t* __restrict__
 
 constexpr uint32_t kDenseBlock = 256;  // frontier vertices per 4096 that pay for staging offsets
 constexpr uint64_t kFusedMaxBlocks = 1024;     // LDS staging: four workgroups per CU
-// degree array, two passes: fewer workgroups take fewer queue atomics
-// (SSSP s24 per query: 512 / 1024 / 2048 workgroups 4.28-4.30 / 4.19-4.24 /
-// 4.35 ms; the one-pass form with 2048: 4.33-4.35 ms)
-constexpr uint64_t kFusedMaxBlocksDeg = 1024;
 // each workgroup of the fused compaction writes one statistics partial
-static_assert(kFusedMaxBlocks <= kStatsMaxBlocks && kFusedMaxBlocksDeg <= kStatsMaxBlocks,
+static_assert(kFusedMaxBlocks <= kStatsMaxBlocks,
               "the partials buffer (stats_parts_needed) holds kStatsMaxBlocks + 1 entries");
 
 // Statistics the compaction counts while it reads the frontier's offsets.
@@ -929,19 +916,60 @@ struct CompactAcc {
 // word, or in `in` when the workgroup has more strides than it caches).  A
 // vertex queued in chunks has its record cleared here; its chunks raise it
 // to the largest value they read.
-constexpr int kFewBits = 4;
 constexpr int kPre = 4;
-constexpr int kDegRow = (int)kSliceBits + 1;  // odd stride: lanes' rows on distinct banks
+// Shapes of the fused compaction with the degree array.  It is bound by
+// dependent round trips (words, degrees and values, queue ranges, placing),
+// so a lane takes 4 vertices (kFineBits) instead of 16 as long as a chip of
+// workgroups covers the graph in the kPre strides it caches; and by the three
+// queue atomics of each workgroup on one line (16 ns a workgroup), so
+// workgroups have 1024 threads and number kFusedBlocks at most, except on
+// graphs that 256 threads each cover too (wavefronts that start and meet
+// sooner).  Per SSSP query, 16 vertices a lane in at most 1024 workgroups of
+// 256 -> these shapes: 12 k vertices 273 -> 219 us, 60 k 420 -> 335, R-MAT s16
+// 417 -> 340, s18 496 -> 436, 1 M 946 -> 841, s21 1202 -> 1095, s22 1712 -> 1623,
+// s24 4000 -> 3905 (with wave.hpp's sums for shuffles in all of these, a third
+// of it); 1 M with workgroups of 256 / 512: 889 / 859, 12 k with 1024: 226.
+constexpr uint32_t kFineBits = 4;
+constexpr int kFusedBlock = 1024;
+constexpr uint64_t kFusedBlocks = 256;
+struct CompactShape {
+  bool fine, small;  // slices of kFineBits; workgroups of kBlock
+  unsigned blocks, block;
+};
+inline CompactShape compact_shape(uint64_t words, bool deg) {
+  const uint64_t lanes = words * (64 / kFineBits);
+  CompactShape c{};
+  c.fine = deg && lanes <= kPre * kFusedBlocks * kFusedBlock;
+  c.small = c.fine && lanes <= kFusedBlocks * kBlock;
+  c.block = deg && !c.small ? kFusedBlock : kBlock;
+  const uint64_t n = ((c.fine ? lanes : words * kSlicesPerWord) + c.block - 1) / c.block;
+  c.blocks = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(n, deg ? kFusedBlocks : kFusedMaxBlocks));
+  return c;
+}
+template <uint32_t SB, int NB>
 __device__ __forceinline__ void compact_frontier_deg(uint64_t* in, uint64_t* __restrict__ out,
                                                      uint64_t words, const DevGraph& g, const Bins& bins,
                                                      uint32_t* __restrict__ q_small, uint32_t* __restrict__ q_med,
                                                      uint64_t* __restrict__ q_chunk, DevStats* __restrict__ st,
                                                      const uint32_t* __restrict__ val, const HubDefer& hub,
                                                      bool queue, CompactAcc& a) {
-  __shared__ uint32_t s_tot[kWavesPerBlock][3];
-  __shared__ uint32_t s_base[kWavesPerBlock][3];
-  __shared__ uint32_t s_deg[kWavesPerBlock][kWave * kDegRow];
-  __shared__ WaveHubs s_hubs[kWavesPerBlock];
+  constexpr int kWaves = NB / kWave;
+  constexpr uint64_t kSpw = 64 / SB;   // slices per word
+  constexpr int kFew = SB / 4;
+  constexpr int kDegRow = (int)SB + 1;  // odd stride: lanes' rows on distinct banks
+  auto slice_bits = [](uint64_t word, uint64_t si) {
+    return (uint32_t)(word >> (SB * (si % kSpw))) & ((1u << SB) - 1u);
+  };
+  auto join_slices = [](uint32_t bits, uint64_t si) {
+    uint64_t w = (uint64_t)bits << (SB * (si % kSpw));
+#pragma unroll
+    for (int d = 1; d < (int)kSpw; d <<= 1) w |= __shfl_xor(w, d, kWave);
+    return w;
+  };
+  __shared__ uint32_t s_tot[kWaves][3];
+  __shared__ uint32_t s_base[kWaves][3];
+  __shared__ uint32_t s_deg[kWaves][kWave * kDegRow];
+  __shared__ WaveHubs s_hubs[kWaves];
   WaveHubs& hubs = s_hubs[wave_id()];
   uint32_t* const drow = &s_deg[wave_id()][lane_id() * kDegRow];
   uint32_t thr = 0xFFFFFFFFu;
@@ -949,18 +977,23 @@ __device__ __forceinline__ void compact_frontier_deg(uint64_t* in, uint64_t* __r
     const uint64_t t = (uint64_t)st->min_val + hub.delta;
     thr = t > 0xFFFFFFFFull ? 0xFFFFFFFFu : (uint32_t)t;
   }
-  const uint64_t slices = words * kSlicesPerWord;
-  const uint64_t stride = (uint64_t)gridDim.x * kBlock;
+  const uint64_t slices = words * kSpw;
+  const uint64_t stride = (uint64_t)gridDim.x * NB;
   // calls f(v, deg) for the vertices of the lane's slice si in `bits`
   auto each = [&](uint64_t si, uint32_t bits, auto&& f) {
-    const uint64_t vbase = si * kSliceBits;
-    if (__popc(bits) > kFewBits) {
+    const uint64_t vbase = si * SB;
+    if (__popc(bits) > kFew) {
       const uint4* p = reinterpret_cast<const uint4*>(g.deg + vbase);
-      const uint4 d0 = p[0], d1 = p[1], d2 = p[2], d3 = p[3];
-      const uint32_t d[16] = {d0.x, d0.y, d0.z, d0.w, d1.x, d1.y, d1.z, d1.w,
-                              d2.x, d2.y, d2.z, d2.w, d3.x, d3.y, d3.z, d3.w};
+      uint4 d[SB / 4];
 #pragma unroll
-      for (int k = 0; k < 16; ++k) drow[k] = d[k];
+      for (int k = 0; k < (int)SB / 4; ++k) d[k] = p[k];
+#pragma unroll
+      for (int k = 0; k < (int)SB / 4; ++k) {
+        drow[4 * k] = d[k].x;
+        drow[4 * k + 1] = d[k].y;
+        drow[4 * k + 2] = d[k].z;
+        drow[4 * k + 3] = d[k].w;
+      }
       for (; bits; bits &= bits - 1) {
         const uint32_t j = (uint32_t)__builtin_ctz(bits);
         f((uint32_t)(vbase + j), (uint64_t)drow[j]);
@@ -980,14 +1013,14 @@ __device__ __forceinline__ void compact_frontier_deg(uint64_t* in, uint64_t* __r
   // loaded together (kPre loads in flight per lane instead of one), and when
   // the workgroup has at most kPre strides the placing pass takes the words
   // from registers instead of reading them again.
-  const uint64_t base0 = blockIdx.x * (uint64_t)kBlock;
+  const uint64_t base0 = blockIdx.x * (uint64_t)NB;
   const uint64_t nstr = base0 < slices ? (slices - base0 + stride - 1) / stride : 0;  // block-uniform
   const bool cached = nstr <= (uint64_t)kPre;
   auto load_words = [&](uint64_t s0, uint64_t (&w)[kPre]) {
 #pragma unroll
     for (int j = 0; j < kPre; ++j) {
       const uint64_t si = base0 + (s0 + j) * stride + threadIdx.x;
-      w[j] = s0 + j < nstr && si < slices ? in[si / kSlicesPerWord] : 0ull;
+      w[j] = s0 + j < nstr && si < slices ? in[si / kSpw] : 0ull;
     }
   };
   uint64_t keep[kPre] = {};  // the cached words, dropped vertices removed
@@ -1001,19 +1034,19 @@ __device__ __forceinline__ void compact_frontier_deg(uint64_t* in, uint64_t* __r
     for (int j = 0; j < kPre; ++j) {
       if (s0 + j >= nstr) break;  // block-uniform
       const uint64_t si = base0 + (s0 + j) * stride + threadIdx.x;
-      const uint64_t wi = si / kSlicesPerWord;
+      const uint64_t wi = si / kSpw;
       const uint32_t word = slice_bits(fulls[j], si);
       uint32_t wait = 0, drop = 0;
       // a dense slice wholly below V takes the drop test of its 16 vertices
       // from four 16-byte loads of the values and four of the propagated
       // values instead of two scalar loads per active vertex
-      const bool vec_drop = drops && __popc(word) > kFewBits && (si + 1) * kSliceBits <= (uint64_t)g.V;
+      const bool vec_drop = drops && __popc(word) > kFew && (si + 1) * SB <= (uint64_t)g.V;
       uint32_t dmask = 0;
       if (vec_drop) {
-        const uint4* pv = reinterpret_cast<const uint4*>(val + si * kSliceBits);
-        const uint4* px = reinterpret_cast<const uint4*>(g.xval + si * kSliceBits);
+        const uint4* pv = reinterpret_cast<const uint4*>(val + si * SB);
+        const uint4* px = reinterpret_cast<const uint4*>(g.xval + si * SB);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 0; q < (int)SB / 4; ++q) {
           const uint4 x = pv[q], r = px[q];
           dmask |= ((r.x != 0u && r.x - 1u == x.x) ? 1u : 0u) << (4 * q);
           dmask |= ((r.y != 0u && r.y - 1u == x.y) ? 2u : 0u) << (4 * q);
@@ -1025,7 +1058,7 @@ __device__ __forceinline__ void compact_frontier_deg(uint64_t* in, uint64_t* __r
         uint32_t x = 0;
         bool have_x = false;
         if (drops && deg != 0) {
-          const uint32_t bit = 1u << (v - si * kSliceBits);
+          const uint32_t bit = 1u << (v - si * SB);
           if (vec_drop) {
             if (dmask & bit) {
               drop |= bit;
@@ -1048,7 +1081,7 @@ __device__ __forceinline__ void compact_frontier_deg(uint64_t* in, uint64_t* __r
           return;
         }
         if (hub.degree && deg >= hub.degree && (have_x ? x : (x = val[v])) >= thr) {
-          wait |= 1u << (v - si * kSliceBits);
+          wait |= 1u << (v - si * SB);
           wait_min = x < wait_min ? x : wait_min;
           ++a.n_def;
           a.m_def += deg;
@@ -1060,12 +1093,12 @@ __device__ __forceinline__ void compact_frontier_deg(uint64_t* in, uint64_t* __r
       });
       a.c_act += (uint32_t)__popc(word & ~drop);
       const uint64_t wait_word = join_slices(wait, si);
-      if (si < slices && si % kSlicesPerWord == 0) out[wi] = wait_word;
+      if (si < slices && si % kSpw == 0) out[wi] = wait_word;
       uint64_t kept = fulls[j];
       if (drops) {
         kept &= ~join_slices(drop, si);
         // read back by the placing pass after the workgroup's barriers
-        if (!cached && kept != fulls[j] && si % kSlicesPerWord == 0) in[wi] = kept;
+        if (!cached && kept != fulls[j] && si % kSpw == 0) in[wi] = kept;
       }
       keep[j] = kept;
     }
@@ -1087,15 +1120,15 @@ __device__ __forceinline__ void compact_frontier_deg(uint64_t* in, uint64_t* __r
   if (threadIdx.x < 3) {
     const int q = threadIdx.x;
     uint32_t tot = 0;
-    for (int w = 0; w < kWavesPerBlock; ++w) { s_base[w][q] = tot; tot += s_tot[w][q]; }
+    for (int w = 0; w < kWaves; ++w) { s_base[w][q] = tot; tot += s_tot[w][q]; }
     uint32_t b = 0;
     if (tot) b = atomicAdd(q == 0 ? &st->n_small : (q == 1 ? &st->n_med : &st->n_chunk), tot);
-    for (int w = 0; w < kWavesPerBlock; ++w) s_base[w][q] += b;
+    for (int w = 0; w < kWaves; ++w) s_base[w][q] += b;
   }
   __syncthreads();
   uint32_t any = 0;
 #pragma unroll
-  for (int w = 0; w < kWavesPerBlock; ++w) any |= s_tot[w][0] | s_tot[w][1] | s_tot[w][2];
+  for (int w = 0; w < kWaves; ++w) any |= s_tot[w][0] | s_tot[w][1] | s_tot[w][2];
   if (!any) return;  // uniform: nothing to place
   // pass 2: the same slices, placed
   uint32_t b_small = s_base[wave_id()][0] + o_small;
@@ -1127,7 +1160,7 @@ __device__ __forceinline__ void compact_frontier_deg(uint64_t* in, uint64_t* __r
   write_hub_chunks(q_chunk, hubs);  // the wavefront's own list
 }
 
-template <bool DEG>
+template <bool DEG, uint32_t SB = (uint32_t)kSliceBits, int NB = kBlock>
 __device__ __forceinline__ void compact_frontier(uint64_t* in, uint64_t* __restrict__ out,
                                                  uint64_t words, const DevGraph& g, const Bins& bins,
                                                  uint32_t* __restrict__ q_small, uint32_t* __restrict__ q_med,
@@ -1135,7 +1168,7 @@ __device__ __forceinline__ void compact_frontier(uint64_t* in, uint64_t* __restr
                                                  const uint32_t* __restrict__ val, const HubDefer& hub, bool queue,
                                                  CompactAcc& a) {
   if constexpr (DEG) {
-    compact_frontier_deg(in, out, words, g, bins, q_small, q_med, q_chunk, st, val, hub, queue, a);
+    compact_frontier_deg<SB, NB>(in, out, words, g, bins, q_small, q_med, q_chunk, st, val, hub, queue, a);
     return;
   }
   __shared__ uint32_t s_tot[kWavesPerBlock][3];
@@ -1264,8 +1297,8 @@ __device__ __forceinline__ void compact_frontier(uint64_t* in, uint64_t* __restr
 // Compaction with the frontier statistics folded in (the GPU and learned
 // schedules' SSSP / CC iterations), so the frontier and its offsets are read
 // once per iteration instead of twice.
-template <bool DEG>
-__global__ __launch_bounds__(kBlock) void k_compact_fused(uint64_t* __restrict__ in,
+template <bool DEG, uint32_t SB = (uint32_t)kSliceBits, int NB = kBlock>
+__global__ __launch_bounds__(NB) void k_compact_fused(uint64_t* __restrict__ in,
                                                           uint64_t* __restrict__ out, uint64_t words, DevGraph g,
                                                           Bins bins, uint32_t* __restrict__ q_small,
                                                           uint32_t* __restrict__ q_med,
@@ -1295,7 +1328,7 @@ __global__ __launch_bounds__(kBlock) void k_compact_fused(uint64_t* __restrict__
     }
   }
   CompactAcc a;
-  compact_frontier<DEG>(in, out, words, g, bins, q_small, q_med, q_chunk, st, val, hub, queue, a);
+  compact_frontier<DEG, SB, NB>(in, out, words, g, bins, q_small, q_med, q_chunk, st, val, hub, queue, a);
   StatsPart p{};
   p.n_active = wave_sum_u32(a.c_act);
   p.m_active = wave_sum_u64(a.m);
@@ -1305,7 +1338,8 @@ __global__ __launch_bounds__(kBlock) void k_compact_fused(uint64_t* __restrict__
   p.min_val = 0xFFFFFFFFu;
   p.n_def = wave_sum_u32(a.n_def);
   p.m_def = wave_sum_u64(a.m_def);
-  stats_block_part(p, parts);
+  if constexpr (NB == kBlock) stats_block_part(p, parts);
+  else stats_wide_part<NB>(p, parts);
 }
 
 // One workgroup behind the expansion of a fused iteration: fixed-order
@@ -1674,8 +1708,8 @@ __global__ __launch_bounds__(kBlock) void k_pull_bfs(DevGraph g, uint32_t* __res
 // frontier among its in-edges, a wavefront writes its word of the next
 // bitmap and counts the vertices found and their out-degrees.
 // Iteration one's front work (frontier {root}) is done by k_init_traverse.
-template <bool DEG>
-__global__ __launch_bounds__(kBlock) void k_bfs_front(const uint64_t* __restrict__ in, uint64_t* __restrict__ out,
+template <bool DEG, uint32_t SB = (uint32_t)kSliceBits, int NB = kBlock>
+__global__ __launch_bounds__(NB) void k_bfs_front(const uint64_t* __restrict__ in, uint64_t* __restrict__ out,
                                                       uint64_t words, DevGraph g, uint64_t E, Bins bins,
                                                       uint32_t* __restrict__ q_small, uint32_t* __restrict__ q_med,
                                                       uint64_t* __restrict__ q_chunk, DevStats* __restrict__ st,
@@ -1736,7 +1770,7 @@ __global__ __launch_bounds__(kBlock) void k_bfs_front(const uint64_t* __restrict
   // (the next run's initialisation clears both bitmaps).
   if (pull || n == 0) return;
   CompactAcc a;
-  compact_frontier<DEG>(const_cast<uint64_t*>(in), out, words, g, bins, q_small, q_med, q_chunk, st, nullptr,
+  compact_frontier<DEG, SB, NB>(const_cast<uint64_t*>(in), out, words, g, bins, q_small, q_med, q_chunk, st, nullptr,
                         HubDefer{0, 1}, true, a);  // nothing dropped without values: `in` is only read
 }
 
@@ -2090,6 +2124,13 @@ uint64_t stats_parts_needed(uint64_t words) {
   return (blocks < kStatsMaxBlocks ? blocks : kStatsMaxBlocks) + 1;
 }
 
+uint64_t fused_parts_needed(uint64_t words) {
+  // the finer slices' count whichever a launch takes, so that one over fewer
+  // words than these has room too
+  const uint64_t blocks = (words * (64 / kFineBits) + kBlock - 1) / kBlock;
+  return (blocks < kStatsMaxBlocks ? blocks : kStatsMaxBlocks) + 1;
+}
+
 int launch_stats(const uint64_t* in, uint64_t* zero_me, uint64_t words, const DevGraph& g, uint64_t E,
                  StatsPart* parts, uint32_t* stripes, RunState* rs, const float* mlp,
                  const uint32_t* val, uint32_t threshold, DevStats* st, DevStats* host_out,
@@ -2126,19 +2167,18 @@ int launch_compact_fused(uint64_t* in, uint64_t* out, uint64_t words, const DevG
                          const uint32_t* val, HubDefer hub, StatsPart* parts, uint32_t* nparts,
                          const RunState* rs, hipStream_t s, const TierTable* choice_tiers) {
   if (hub.degree && (!val || !hub.delta)) return set_error(CG_ERR_INVALID, "hub deferral needs values and delta >= 1");
-  const uint64_t slices = words * kSlicesPerWord;
-  uint64_t blocks = slices ? (slices + kBlock - 1) / kBlock : 1;
-  const uint64_t cap = g.deg ? kFusedMaxBlocksDeg : kFusedMaxBlocks;
-  if (blocks > cap) blocks = cap;
+  const CompactShape sh = compact_shape(words, g.deg != nullptr);
   const TierTable tiers = choice_tiers ? *choice_tiers : TierTable{};
-  if (g.deg)
-    hipLaunchKernelGGL(k_compact_fused<true>, dim3((unsigned)blocks), dim3(kBlock), 0, s, in, out, words, g, bins,
-                       q_small, q_med, q_chunk, st, val, hub, parts, choice_tiers ? 1 : 0, tiers, rs);
-  else
-    hipLaunchKernelGGL(k_compact_fused<false>, dim3((unsigned)blocks), dim3(kBlock), 0, s, in, out, words, g, bins,
-                       q_small, q_med, q_chunk, st, val, hub, parts, choice_tiers ? 1 : 0, tiers, rs);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(sh.blocks), dim3(sh.block), 0, s, in, out, words, g, bins, q_small, q_med,
+                       q_chunk, st, val, hub, parts, choice_tiers ? 1 : 0, tiers, rs);
+  };
+  if (sh.small) launch(k_compact_fused<true, kFineBits>);
+  else if (sh.fine) launch(k_compact_fused<true, kFineBits, kFusedBlock>);
+  else if (g.deg) launch(k_compact_fused<true, (uint32_t)kSliceBits, kFusedBlock>);
+  else launch(k_compact_fused<false>);
   CG_LAUNCH_CHECK();
-  *nparts = (uint32_t)blocks;
+  *nparts = sh.blocks;
   return CG_OK;
 }
 
@@ -2229,16 +2269,15 @@ int launch_bfs_front(const uint64_t* in, uint64_t* out, uint64_t words, const De
                      const Bins& bins, uint32_t* q_small, uint32_t* q_med, uint64_t* q_chunk, DevStats* st,
                      DevStats* st_next, const unsigned long long* cnt_prev, unsigned long long* cnt_cur,
                      const RunState* rs_prev, RunState* rs_cur, DevStats* host_out, hipStream_t s) {
-  const uint64_t slices = words * kSlicesPerWord;
-  uint64_t fblocks = slices ? (slices + kBlock - 1) / kBlock : 1;
-  const uint64_t cap = g.deg ? kFusedMaxBlocksDeg : kFusedMaxBlocks;
-  if (fblocks > cap) fblocks = cap;
-  if (g.deg)
-    hipLaunchKernelGGL(k_bfs_front<true>, dim3((unsigned)fblocks), dim3(kBlock), 0, s, in, out, words, g, E, bins,
-                       q_small, q_med, q_chunk, st, st_next, cnt_prev, cnt_cur, rs_prev, rs_cur, host_out);
-  else
-    hipLaunchKernelGGL(k_bfs_front<false>, dim3((unsigned)fblocks), dim3(kBlock), 0, s, in, out, words, g, E, bins,
-                       q_small, q_med, q_chunk, st, st_next, cnt_prev, cnt_cur, rs_prev, rs_cur, host_out);
+  const CompactShape sh = compact_shape(words, g.deg != nullptr);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(sh.blocks), dim3(sh.block), 0, s, in, out, words, g, E, bins, q_small, q_med,
+                       q_chunk, st, st_next, cnt_prev, cnt_cur, rs_prev, rs_cur, host_out);
+  };
+  if (sh.small) launch(k_bfs_front<true, kFineBits>);
+  else if (sh.fine) launch(k_bfs_front<true, kFineBits, kFusedBlock>);
+  else if (g.deg) launch(k_bfs_front<true, (uint32_t)kSliceBits, kFusedBlock>);
+  else launch(k_bfs_front<false>);
   CG_LAUNCH_CHECK();
   return CG_OK;
 }
