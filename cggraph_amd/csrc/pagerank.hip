@@ -111,10 +111,10 @@ struct PrPlan {
   DevBuf<uint32_t> pb_t2_multi;         // tile's bin is cut into several tiles
   DevBuf<unsigned long long> pb_sum;    // fixed-point sums of the bins cut into several tiles
   // propagation blocking over (source, bin) pairs (layout 5): pb_ent and
-  // pb_val hold one entry per pair, pb_dloc one per edge (destination within
-  // its bin | 0x8000 on a pair's first edge), pb_gbase the pair of every 64th
+  // pb_val hold one entry per pair, pb_dloc one per edge (8 * destination
+  // within its bin | 4 on a pair's first edge), pb_pair the pair of every 8th
   // edge; the graph is renumbered by descending out-degree (perm)
-  DevBuf<uint32_t> pb_gbase;
+  DevBuf<uint32_t> pb_pair;
   uint64_t pb_pairs = 0;
   // bins cut into several gather tiles: each tile writes its 8192 sums to a
   // row of its own (pb_t2_multi = row + 1), bin i's rows are
@@ -590,14 +590,19 @@ __global__ void k_row_ranges(const uint64_t* __restrict__ off, const uint32_t* _
   }
 }
 
-// The sum of a row is complete: LAST leaves the rank at the caller's id of
-// the row, the other sweeps leave what the next one gathers.
+// Rank r of vertex v: LAST leaves it at the caller's id of the vertex, the
+// other sweeps leave what the next one gathers.
+template <bool LAST>
+__device__ __forceinline__ void put_rank(uint32_t v, float r, uint32_t deg, const uint32_t* __restrict__ perm,
+                                         float* __restrict__ out) {
+  if constexpr (LAST) out[perm ? perm[v] : v] = r;
+  else out[v] = deg ? r / (float)deg : 0.0f;
+}
+
 template <bool LAST>
 __device__ __forceinline__ void row_done(uint32_t v, double sum, uint32_t deg, float base, float damping,
                                          const uint32_t* __restrict__ perm, float* __restrict__ out) {
-  const float r = (float)(base + damping * sum);
-  if constexpr (LAST) out[perm ? perm[v] : v] = r;
-  else out[v] = deg ? r / (float)deg : 0.0f;
+  put_rank<LAST>(v, (float)(base + damping * sum), deg, perm, out);
 }
 
 template <bool LAST>
@@ -1514,42 +1519,37 @@ int build_blocked(const DevGraph& g, uint64_t E, PrPlan* p, hipStream_t s) {
 //
 // An edge's contribution is its source's, so the edges of one source into one
 // bin carry the same value.  Writing and reading it once per (source, bin)
-// pair instead of once per edge leaves a pass of 2 bytes per edge (the
-// destination) plus 12 bytes per pair.  On a graph renumbered by descending
+// pair instead of once per edge leaves a pass of 2.5 bytes per edge (the
+// destination, and the pair of every eighth) plus 12 bytes per pair.  On a graph renumbered by descending
 // out-degree the hot destinations share few bins, so the pairs are few:
 // R-MAT edge factor 44 has 0.08 / 0.13 / 0.18 pairs per edge at scale
 // 18 / 20 / 22 (8192-vertex bins), against 1 per edge before.
 //   scatter  k_pb_scatter over the pairs' chunk-major entries (source within
 //            its chunk | bin << 13): one store per pair into its bin-major slot;
-//   gather   k_pbp_gather: a wavefront takes 256 consecutive edges of a bin
-//            (four per lane, one 8-byte load); the pair of each edge is the
-//            group's first pair (pb_gbase) plus the pair starts (0x8000
-//            flags) before it, counted from one ballot per edge slot; its value is
-//            one load from the pair's slot (neighbouring edges share pairs,
-//            so these loads hit the same lines), added in 64-bit fixed point
-//            into the bin's LDS sums.
+//   gather   k_pbp_gather: a wavefront takes 512 consecutive edges of a bin
+//            (eight per lane, one 16-byte load); a lane's first edge has its
+//            pair in pb_pair and each flagged edge (the first of a pair) moves
+//            on to the next; its value is one load from the pair's slot
+//            (neighbouring edges share pairs, so these loads hit the same
+//            lines), added in 64-bit fixed point into the bin's LDS sums.
 // Pairs inside one (chunk, bin) run are ordered by source in both orders
 // (a radix sort on (chunk, bin, source)), so one delta per run maps a pair's
 // chunk-major index to its bin-major one, as for the edges of layout 4.
-constexpr int kPpEdges = 4;                       // edges per lane in a group (one 8-byte load)
-constexpr int kPpGroupShift = 8;                  // edges per group: 64 lanes x kPpEdges = 2^8
+constexpr int kPpEdges = 8;                       // edges per lane in a group (one 16-byte load)
+constexpr int kPpGroupShift = 9;                  // edges per group: 64 lanes x kPpEdges = 2^9
 constexpr uint64_t kPpGroup = 1ull << kPpGroupShift;
-// Gather shape, measured at R-MAT s25 / ef44 (ms per iteration): workgroups
-// of 256 / 512 / 1024 threads with 16 / 8 / 2 groups in flight per wavefront
-// 4.85-4.90 / 3.60-3.63 / 2.89-2.91; at 1024 threads 1 / 3 / 4 groups
-// 2.92-2.95 / 3.77-3.85 / 3.81-3.84 (three groups and more need more than the
-// 64 registers that eight wavefronts per SIMD leave); tiles of 2^18 / 2^19 /
-// 2^20 edges 3.05 / 2.89-2.91 / 2.79-2.91.  The LDS sums (64 KB) allow two
-// workgroups per CU, so the workgroup size sets the wavefronts per SIMD.
-constexpr int kPpGroups = 2;                      // groups in flight per wavefront
+// Gather: bound by its instructions.  It was 27 vector instructions per edge
+// (a ballot and a count of pair starts per edge slot, a conversion of seven,
+// 64-bit addresses) and 1.98 ms of a sweep at R-MAT s25 / ef44; the pair of
+// every eighth edge, flags and destinations that are byte offsets, 32-bit
+// addresses from the group's first pair and the conversion below leave 8, and
+// 1.24 ms (4.9 GB read: 4 TB/s).  The LDS sums (64 KB) allow two workgroups
+// per CU, so the workgroup size sets the wavefronts per SIMD; 1 / 2 / 3 groups
+// in flight per wavefront 41.7 / 42.8 / 44 ms for twenty sweeps.
+constexpr int kPpGroups = 1;                      // groups in flight per wavefront
 constexpr int kPpBlock = 1024;                    // gather workgroup: 16 wavefronts share the LDS sums
 constexpr uint64_t kPpBinTile = 1ull << 20;       // gather: edges per workgroup
 constexpr uint64_t kPpPad = 2 * kPpGroup;         // zero entries past the last edge
-
-// set bits of m below this lane (v_mbcnt)
-__device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
-  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-}
 
 __global__ void k_pp_flags(const uint64_t* __restrict__ off, const uint32_t* __restrict__ dst,
                            const uint32_t* __restrict__ src, uint64_t E, uint32_t* __restrict__ flags) {
@@ -1601,12 +1601,12 @@ __global__ void k_pp_place(const uint64_t* __restrict__ key, const uint32_t* __r
 __global__ void k_pp_edges(const uint32_t* __restrict__ dst, const uint32_t* __restrict__ incl, uint64_t E,
                            const uint64_t* __restrict__ pfirst, const uint32_t* __restrict__ bm_of,
                            const uint64_t* __restrict__ eoff, uint16_t* __restrict__ dloc,
-                           uint32_t* __restrict__ gbase) {
+                           uint32_t* __restrict__ pair) {
   for (uint64_t e = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; e < E; e += (uint64_t)gridDim.x * blockDim.x) {
     const uint32_t sm = incl[e] - 1, j = bm_of[sm];
     const uint64_t k = e - pfirst[sm], pos = eoff[j] + k;
-    dloc[pos] = (uint16_t)((dst[e] & (kPbSize - 1)) | (k == 0 ? 0x8000u : 0u));
-    if ((pos & (kPpGroup - 1)) == 0) gbase[pos >> kPpGroupShift] = j;
+    dloc[pos] = (uint16_t)((dst[e] & (kPbSize - 1)) << 3 | (k == 0 ? 4u : 0u));
+    if (pos % kPpEdges == 0) pair[pos / kPpEdges] = j;
   }
 }
 
@@ -1617,70 +1617,100 @@ __global__ void k_pp_bin_edges(const uint64_t* __restrict__ bin_off, const uint6
     out[b] = eoff[bin_off[b]];
 }
 
+// x * 2^56, rounded as to_fixed does, for 0 <= x < 2^-4: adding 2^-4 in 64
+// bits leaves a last place of 2^-56, so the mantissa is the result.  Three
+// instructions instead of the conversion's seven.
+constexpr uint32_t kSmallBits = 0x3D800000u;  // 2^-4; floats of larger bits are larger, negative or NaN
+__device__ __forceinline__ unsigned long long to_fixed_small(float x) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong((double)x + 0x1p-4);
+  return b - 0x3FB0000000000000ull;
+}
+
+template <bool LAST>
 __global__ __launch_bounds__(kPpBlock) void k_pbp_gather(const float* __restrict__ val,
                                                          const uint16_t* __restrict__ dloc,
-                                                         const uint32_t* __restrict__ gbase,
+                                                         const uint32_t* __restrict__ pair,
                                                          const uint32_t* __restrict__ t_bin,
                                                          const uint64_t* __restrict__ t_lo,
                                                          const uint64_t* __restrict__ t_hi,
                                                          const uint32_t* __restrict__ t_multi, uint32_t V,
                                                          const uint32_t* __restrict__ deg, float base,
                                                          float damping, unsigned long long* __restrict__ rows,
-                                                         float* __restrict__ rank, float* __restrict__ contrib) {
+                                                         const uint32_t* __restrict__ perm, float* __restrict__ out) {
   __shared__ unsigned long long acc[kPbSize];
   const uint32_t t = blockIdx.x;
   for (uint32_t k = threadIdx.x; k < kPbSize; k += kPpBlock) acc[k] = 0;
   __syncthreads();
   const uint64_t lo = t_lo[t], hi = t_hi[t];
   if (hi > lo) {
-    // a group is 2^8 consecutive edges, four per lane (lane l: 4l .. 4l + 3);
-    // an edge's pair is the group's first pair plus the pair starts (0x8000
-    // flags) after the group's first edge up to it: per edge slot k, a
-    // ballot of the flags; the lanes below count with v_mbcnt
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    // a group is 2^9 consecutive edges, eight per lane; the lane's first edge
+    // belongs to pair[] and each flag moves on to the next pair
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     constexpr uint32_t kWaves = kPpBlock / 64;
-    const uint64_t* dl4 = reinterpret_cast<const uint64_t*>(dloc);
+    const u32x4* dl = reinterpret_cast<const u32x4*>(dloc);
     const uint64_t g0 = lo >> kPpGroupShift, g1 = (hi - 1) >> kPpGroupShift;  // inclusive
+    // the sums' byte offset of the lane's k-th edge, and 4 on a pair's first
+    auto slot = [](const u32x4& d, int k) { return k & 1 ? d[k / 2] >> 16 & 0xFFF8u : d[k / 2] & 0xFFF8u; };
+    auto step = [](const u32x4& d, int k) { return k & 1 ? d[k / 2] >> 16 & 4u : d[k / 2] & 4u; };
+    auto add = [&](uint32_t at, unsigned long long x) {
+      atomicAdd(reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(acc) + at), x);
+    };
     for (uint64_t g = g0 + wave; g <= g1; g += (uint64_t)kPpGroups * kWaves) {
-      uint64_t dd[kPpGroups];
-      uint32_t gb[kPpGroups];
+      if ((g << kPpGroupShift) >= lo && ((g + (kPpGroups - 1) * kWaves + 1) << kPpGroupShift) <= hi) {
+        u32x4 d[kPpGroups];
+        uint32_t at[kPpGroups];
 #pragma unroll
+        for (int u = 0; u < kPpGroups; ++u) {
+          const uint64_t i = (g + (uint64_t)u * kWaves) * 64 + lane;
+          d[u] = dl[i];
+          at[u] = pair[i];
+        }
+        float x[kPpGroups][kPpEdges];
+        uint32_t largest = 0;
+#pragma unroll
+        for (int u = 0; u < kPpGroups; ++u) {
+          // 32-bit byte offsets from the group's first pair
+          const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)at[u]);
+          const char* v = reinterpret_cast<const char*>(val + first);
+          uint32_t o = (at[u] - first) * 4;
+#pragma unroll
+          for (int k = 0; k < kPpEdges; ++k) {
+            if (k) o += step(d[u], k);
+            x[u][k] = *reinterpret_cast<const float*>(v + o);
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < kPpGroups; ++u)
+#pragma unroll
+          for (int k = 0; k < kPpEdges; ++k) {
+            const uint32_t b = __float_as_uint(x[u][k]);
+            largest = largest > b ? largest : b;
+          }
+        if (__ballot(largest >= kSmallBits)) {
+#pragma unroll
+          for (int u = 0; u < kPpGroups; ++u)
+#pragma unroll
+            for (int k = 0; k < kPpEdges; ++k) add(slot(d[u], k), to_fixed(x[u][k]));
+        } else {
+#pragma unroll
+          for (int u = 0; u < kPpGroups; ++u)
+#pragma unroll
+            for (int k = 0; k < kPpEdges; ++k) add(slot(d[u], k), to_fixed_small(x[u][k]));
+        }
+        continue;
+      }
+      // groups at the tile's ends: only its own edges
       for (int u = 0; u < kPpGroups; ++u) {
         const uint64_t gg = g + (uint64_t)u * kWaves;
-        const bool ok = gg <= g1;
-        dd[u] = ok ? dl4[gg * 64 + lane] : 0ull;
-        gb[u] = ok ? gbase[gg] : 0u;
-      }
-      float x[kPpGroups * kPpEdges];
-#pragma unroll
-      for (int u = 0; u < kPpGroups; ++u) {
-        uint32_t pi = gb[u];
-        uint32_t f[kPpEdges];
+        if (gg > g1) break;
+        const u32x4 d = dl[gg * 64 + lane];
+        uint64_t pi = pair[gg * 64 + lane];
+        const uint64_t e0 = (gg << kPpGroupShift) + kPpEdges * lane;
 #pragma unroll
         for (int k = 0; k < kPpEdges; ++k) {
-          f[k] = (uint32_t)(dd[u] >> (16 * k + 15)) & 1u;
-          uint64_t b = __ballot(f[k] != 0);
-          if (k == 0) b &= ~1ull;  // the group's first edge belongs to pair gb
-          pi += lanes_below(b);
-        }
-        if (lane == 0) f[0] = 0;
-        const uint64_t gg = g + (uint64_t)u * kWaves, e0 = (gg << kPpGroupShift) + 4 * lane;
-        const bool whole = gg <= g1 && (gg << kPpGroupShift) >= lo && ((gg + 1) << kPpGroupShift) <= hi;  // uniform
-#pragma unroll
-        for (int k = 0; k < kPpEdges; ++k) {
-          pi += f[k];
-          const bool in = whole || (gg <= g1 && e0 + k >= lo && e0 + k < hi);
-          x[u * kPpEdges + k] = in ? val[pi] : 0.0f;
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < kPpGroups; ++u) {
-        const uint64_t gg = g + (uint64_t)u * kWaves, e0 = (gg << kPpGroupShift) + 4 * lane;
-        const bool whole = gg <= g1 && (gg << kPpGroupShift) >= lo && ((gg + 1) << kPpGroupShift) <= hi;
-#pragma unroll
-        for (int k = 0; k < kPpEdges; ++k) {
-          const bool in = whole || (gg <= g1 && e0 + k >= lo && e0 + k < hi);
-          if (in) atomicAdd(&acc[(uint32_t)(dd[u] >> (16 * k)) & (kPbSize - 1)], to_fixed(x[u * kPpEdges + k]));
+          if (k) pi += step(d, k) >> 2;
+          if (e0 + k >= lo && e0 + k < hi) add(slot(d, k), to_fixed(val[pi]));
         }
       }
     }
@@ -1692,24 +1722,37 @@ __global__ __launch_bounds__(kPpBlock) void k_pbp_gather(const float* __restrict
     for (uint32_t k = threadIdx.x; k < kPbSize; k += kPpBlock) row[k] = acc[k];
   } else {
     for (uint32_t k = threadIdx.x; k < kPbSize && v0 + k < V; k += kPpBlock)
-      finish((uint32_t)(v0 + k), (float)((double)acc[k] * kFixInv), base, damping, deg, rank, contrib);
+      put_rank<LAST>((uint32_t)(v0 + k), base + damping * (float)((double)acc[k] * kFixInv),
+                     LAST ? 0u : deg[v0 + k], perm, out);
   }
 }
 
+constexpr uint32_t kFinishRows = 16;
+
 // Bins cut into several gather tiles: the tiles' rows added up per vertex
 // (in row order), then the ranks.
+template <bool LAST>
 __global__ __launch_bounds__(kBlock) void k_pbp_finish(const uint32_t* __restrict__ bins,
                                                        const uint32_t* __restrict__ mrow, uint32_t V,
                                                        const uint32_t* __restrict__ deg, float base, float damping,
                                                        const unsigned long long* __restrict__ part,
-                                                       float* __restrict__ rank, float* __restrict__ contrib) {
+                                                       const uint32_t* __restrict__ perm, float* __restrict__ out) {
   const uint32_t i = blockIdx.x / (kPbSize / kBlock);
   const uint32_t k = (blockIdx.x % (kPbSize / kBlock)) * kBlock + threadIdx.x;
   const uint64_t v = ((uint64_t)bins[i] << kPbShift) + k;
   if (v >= V) return;
+  // kFinishRows rows in flight: the hottest bin has hundreds, and one after
+  // the other they took 94 us of a sweep at s25 / ef44
   unsigned long long x = 0;
-  for (uint32_t r = mrow[i]; r < mrow[i + 1]; ++r) x += part[(uint64_t)r * kPbSize + k];
-  finish((uint32_t)v, (float)((double)x * kFixInv), base, damping, deg, rank, contrib);
+  const uint32_t r1 = mrow[i + 1];
+  for (uint32_t r = mrow[i]; r < r1; r += kFinishRows) {
+    unsigned long long y[kFinishRows];
+#pragma unroll
+    for (uint32_t j = 0; j < kFinishRows; ++j) y[j] = part[(uint64_t)(r + j < r1 ? r + j : r) * kPbSize + k];
+#pragma unroll
+    for (uint32_t j = 0; j < kFinishRows; ++j) x += r + j < r1 ? y[j] : 0ull;
+  }
+  put_rank<LAST>((uint32_t)v, base + damping * (float)((double)x * kFixInv), LAST ? 0u : deg[v], perm, out);
 }
 
 // Tiles of the two passes: chunk c's pairs [hb[c], hb[c + 1]) in pieces of
@@ -1808,8 +1851,9 @@ int build_pairs(cg_graph* graph, PrPlan* p, hipStream_t s) {
   const uint64_t P = P32;
   p->pb_pairs = P;
   // pairs: entry 4 B read, contribution 4 B written and 4 B read; edges:
-  // 2 B read (+ one 4-byte group pair per 256); per vertex as layout 4
-  p->stream_bytes = 12.0 * (double)P + (2.0 + 4.0 / (double)kPpGroup) * (double)E + 16.0 * (double)V;
+  // 2 B read (+ 4 B per eight); per vertex a degree and a contribution read,
+  // a contribution written
+  p->stream_bytes = 12.0 * (double)P + (2.0 + 4.0 / kPpEdges) * (double)E + 12.0 * (double)V;
   p->pb_narrow = P < (1ull << 31);
   // the pairs in source-major order, and the pairs of every (chunk, bin) run
   const uint64_t cells = (uint64_t)nc * nb;
@@ -1885,10 +1929,10 @@ int build_pairs(cg_graph* graph, PrPlan* p, hipStream_t s) {
   // the edges: destination within its bin, flagged at each pair's first edge;
   // zero entries past the end keep a tile's last group in bounds
   CG_TRY(p->pb_dloc.ensure(E + kPpPad));
-  CG_TRY(p->pb_gbase.ensure((E + kPpGroup - 1) / kPpGroup + 2));
+  CG_TRY(p->pb_pair.ensure((E + kPpPad) / kPpEdges));
   CG_HIP(hipMemsetAsync(p->pb_dloc.p + E, 0, kPpPad * sizeof(uint16_t), s));
   hipLaunchKernelGGL(k_pp_edges, dim3(grid_of(E)), dim3(kBlock), 0, s, g.dst, incl.p, E, pfirst.p, bm_of.p, eoff.p,
-                     p->pb_dloc.p, p->pb_gbase.p);
+                     p->pb_dloc.p, p->pb_pair.p);
   PR_LAUNCH_OK();
   DevBuf<uint64_t> bin_edges;
   CG_TRY(bin_edges.ensure((uint64_t)nb + 1));
@@ -2029,9 +2073,9 @@ int pr_run(const DevGraph& g, PrPlan* plan, int iters, float damping, float* ran
                           : Csc{g.in_off, g.in_src, plan->deg.p, V, nullptr};
   const uint64_t plan_edges = plan->edges;
   // the ranks alternate between two buffers and end in the caller's; the row
-  // blocks write them there in the last sweep only
-  const bool rows = plan->rows.n != 0;
-  const bool swapped = !rows && (iters + (relabel ? 1 : 0)) % 2;
+  // blocks and the pairs write them there in the last sweep only
+  const bool pairs = plan->layout == kLayoutPairs, direct = pairs || plan->rows.n != 0;
+  const bool swapped = !direct && (iters + (relabel ? 1 : 0)) % 2;
   float* r_cur = swapped ? tmp_rank : rank;
   float* r_nxt = swapped ? rank : tmp_rank;
   float* c_cur = contrib;
@@ -2059,21 +2103,25 @@ int pr_run(const DevGraph& g, PrPlan* plan, int iters, float damping, float* ran
                              plan->pb_t1_chunk.p, plan->pb_t1_lo.p, plan->pb_t1_hi.p, plan->pb_nb, V,
                              plan->pb_delta.p, c_cur, plan->pb_val.p);
       }
-      if (plan->layout == kLayoutPairs)
-        hipLaunchKernelGGL(k_pbp_gather, dim3(plan->pb_t2), dim3(kPpBlock), 0, s, plan->pb_val.p, plan->pb_dloc.p,
-                           plan->pb_gbase.p, plan->pb_t2_bin.p, plan->pb_t2_lo.p, plan->pb_t2_hi.p,
-                           plan->pb_t2_multi.p, V, plan->deg.p, base, damping, plan->pb_part.p, r_nxt, c_nxt);
-      else
+      if (pairs) {
+        const bool last = it + 1 == iters;
+        float* out = last ? rank : c_nxt;
+        hipLaunchKernelGGL(last ? k_pbp_gather<true> : k_pbp_gather<false>, dim3(plan->pb_t2), dim3(kPpBlock), 0, s,
+                           plan->pb_val.p, plan->pb_dloc.p, plan->pb_pair.p, plan->pb_t2_bin.p, plan->pb_t2_lo.p,
+                           plan->pb_t2_hi.p, plan->pb_t2_multi.p, V, plan->deg.p, base, damping, plan->pb_part.p,
+                           plan->perm.p, out);
+        if (plan->pb_multi)
+          hipLaunchKernelGGL(last ? k_pbp_finish<true> : k_pbp_finish<false>,
+                             dim3(plan->pb_multi * (kPbSize / kBlock)), dim3(kBlock), 0, s, plan->pb_multi_bins.p,
+                             plan->pb_mrow.p, V, plan->deg.p, base, damping, plan->pb_part.p, plan->perm.p, out);
+      } else {
         hipLaunchKernelGGL(k_pb_gather, dim3(plan->pb_t2), dim3(kBlock), 0, s, plan->pb_val.p, plan->pb_dloc.p,
                            plan->pb_t2_bin.p, plan->pb_t2_lo.p, plan->pb_t2_hi.p, plan->pb_t2_multi.p, V,
                            plan->deg.p, base, damping, plan->pb_sum.p, r_nxt, c_nxt);
-      if (plan->pb_multi && plan->layout == kLayoutPairs)
-        hipLaunchKernelGGL(k_pbp_finish, dim3(plan->pb_multi * (kPbSize / kBlock)), dim3(kBlock), 0, s,
-                           plan->pb_multi_bins.p, plan->pb_mrow.p, V, plan->deg.p, base, damping, plan->pb_part.p,
-                           r_nxt, c_nxt);
-      else if (plan->pb_multi)
-        hipLaunchKernelGGL(k_pb_finish, dim3(plan->pb_multi * (kPbSize / kBlock)), dim3(kBlock), 0, s,
-                           plan->pb_multi_bins.p, V, plan->deg.p, base, damping, plan->pb_sum.p, r_nxt, c_nxt);
+        if (plan->pb_multi)
+          hipLaunchKernelGGL(k_pb_finish, dim3(plan->pb_multi * (kPbSize / kBlock)), dim3(kBlock), 0, s,
+                             plan->pb_multi_bins.p, V, plan->deg.p, base, damping, plan->pb_sum.p, r_nxt, c_nxt);
+      }
     } else if (plan->layout == kLayoutSegmented) {
       for (uint32_t w = 0; w < plan->nseg; ++w) {
         const uint32_t r0 = plan->seg_run[w], r1 = plan->seg_run[w + 1];
@@ -2122,7 +2170,7 @@ int pr_run(const DevGraph& g, PrPlan* plan, int iters, float damping, float* ran
     std::swap(r_cur, r_nxt);
     std::swap(c_cur, c_nxt);
   }
-  if (relabel && !rows) {
+  if (relabel && !direct) {
     // back to the caller's ids: r_nxt is the caller's buffer after the last swap
     hipLaunchKernelGGL(k_unpermute, dim3(std::min<unsigned>(vblocks, 65536)), dim3(kBlock), 0, s, plan->perm.p,
                        r_cur, V, r_nxt);

@@ -45,3 +45,30 @@ def test_row_blocks(oracle, layout):
             l1 = float(np.abs(r1.astype(np.float64) - ref).sum())
             assert l1 <= 1e-6, (name, iters, l1)
         g.close()
+
+
+def test_pair_groups(oracle):
+    """Pair blocking's gather (layout 5): whole groups of 512 edges and the
+    ends of tiles, contributions either side of 2^-4 (the wide conversion),
+    hot bins in several tiles, ranks in the caller's ids."""
+    rng = np.random.default_rng(9)
+    cases = []
+    for n in (511, 512, 513, 1100):  # everything into vertex 0, which gives half the mass to vertex 1
+        cases.append((n, np.arange(n), np.r_[1, np.zeros(n - 1, np.int64)]))
+    V = 40001  # three bins, the first in several tiles
+    src = (V * rng.random(900001) ** 3).astype(np.int64)
+    dst = np.where(rng.random(900001) < 0.9, rng.integers(0, 8192, 900001), rng.integers(0, V, 900001))
+    cases.append((V, src, dst))
+    for V, src, dst in cases:
+        og = oracle.csr_build(V, src.astype(np.uint32), dst.astype(np.uint32))
+        g = cg.Graph.from_csr(og.offsets, og.dest)
+        for iters in (0, 1, 2, 20):
+            e = cg.Engine(g, PR, pr_layout=5, pr_iterations=iters)
+            r1, _ = e.run()
+            r2, _ = e.run()
+            e.close()
+            assert np.array_equal(r1.view(np.uint32), r2.view(np.uint32)), (V, iters)
+            l1 = float(np.abs(r1.astype(np.float64) - oracle.pagerank64(og, iters, 0.85)).sum())
+            assert l1 <= 1e-6, (V, iters, l1)
+        g.close()
+
