@@ -1548,7 +1548,23 @@ constexpr uint64_t kPpGroup = 1ull << kPpGroupShift;
 // in flight per wavefront 41.7 / 42.8 / 44 ms for twenty sweeps.
 constexpr int kPpGroups = 1;                      // groups in flight per wavefront
 constexpr int kPpBlock = 1024;                    // gather workgroup: 16 wavefronts share the LDS sums
-constexpr uint64_t kPpBinTile = 1ull << 20;       // gather: edges per workgroup
+// Tiles of the two passes.  512 gather workgroups are resident (two per CU),
+// so a tile is at most an even share of the edges; small tiles cut more bins
+// into several, whose sums go through memory (twenty sweeps, ms, tiles of
+// 2^15 / 2^16 / 2^17 / 2^18 / 2^19 / 2^20: 21 x 16 1.7 / 1.6 / 1.8 / 2.2 / 2.4 /
+// 3.6; 22 x 16 - / 3.1 / 3.0 / 3.3 / 3.7 / 5.4; 24 x 16 - / - / - / 10.6 / 10.7 /
+// 12.3; 25 x 44 - / - / - / 46.8 / 45.2 / 41.7).  The scatter loads its chunk's
+// contributions for each tile, so those are not cut below 2^14 pairs.
+inline uint64_t pair_bin_tile(uint64_t E) {
+  uint64_t t = 1ull << 20;
+  while (t > (1ull << 15) && E < t * 480) t >>= 1;
+  return t;
+}
+inline uint64_t pair_chunk_tile(uint64_t P) {
+  uint64_t t = kPbTile;
+  while (t > (1ull << 14) && P < t * 1024) t >>= 1;
+  return t;
+}
 constexpr uint64_t kPpPad = 2 * kPpGroup;         // zero entries past the last edge
 
 __global__ void k_pp_flags(const uint64_t* __restrict__ off, const uint32_t* __restrict__ dst,
@@ -1756,19 +1772,19 @@ __global__ __launch_bounds__(kBlock) void k_pbp_finish(const uint32_t* __restric
 }
 
 // Tiles of the two passes: chunk c's pairs [hb[c], hb[c + 1]) in pieces of
-// kPbTile, bin b's edges [he[b], he[b + 1]) in pieces of bin_tile (every
+// chunk_tile, bin b's edges [he[b], he[b + 1]) in pieces of bin_tile (every
 // bin gets a tile, which writes its ranks even when it has no in-edges).
-int pb_tiles(PrPlan* p, const std::vector<uint64_t>& hb, const std::vector<uint64_t>& he, uint64_t bin_tile,
-             hipStream_t s) {
+int pb_tiles(PrPlan* p, const std::vector<uint64_t>& hb, const std::vector<uint64_t>& he, uint64_t chunk_tile,
+             uint64_t bin_tile, hipStream_t s) {
   const uint32_t nc = (uint32_t)hb.size() - 1, nb = (uint32_t)he.size() - 1;
   std::vector<uint32_t> t1c, t2b, t2m, multi, mrow;
   std::vector<uint64_t> t1l, t1h, t2l, t2h;
   uint32_t rows = 0;
   for (uint32_t c = 0; c < nc; ++c)
-    for (uint64_t lo = hb[c]; lo < hb[c + 1]; lo += kPbTile) {
+    for (uint64_t lo = hb[c]; lo < hb[c + 1]; lo += chunk_tile) {
       t1c.push_back(c);
       t1l.push_back(lo);
-      t1h.push_back(std::min(hb[c + 1], lo + kPbTile));
+      t1h.push_back(std::min(hb[c + 1], lo + chunk_tile));
     }
   for (uint32_t b = 0; b < nb; ++b) {
     const uint64_t n = he[b + 1] - he[b];
@@ -1943,7 +1959,7 @@ int build_pairs(cg_graph* graph, PrPlan* p, hipStream_t s) {
   CG_HIP(hipMemcpyAsync(hb.data(), bounds.p, hb.size() * 8, hipMemcpyDeviceToHost, s));
   CG_HIP(hipMemcpyAsync(he.data(), bin_edges.p, he.size() * 8, hipMemcpyDeviceToHost, s));
   CG_HIP(hipStreamSynchronize(s));
-  return pb_tiles(p, hb, he, kPpBinTile, s);
+  return pb_tiles(p, hb, he, pair_chunk_tile(P), pair_bin_tile(E), s);
 }
 
 template <int P>
@@ -1976,13 +1992,33 @@ int pr_plan_create(cg_graph* graph, uint32_t layout, uint32_t seg_log2, uint32_t
   // pull: 0.30-0.35 vs 0.39-0.43 ms at 2^22, 0.54 vs 0.93 at 2^23; at 2^21
   // the two are within box-to-box spread, 0.17-0.20 vs 0.17 ms, and below it
   // the pull wins: 0.10 vs 0.12-0.16 ms at 2^20)
-  // and over (source, bin) pairs from 2^24 (per iteration, R-MAT: ef16 0.82 vs
-  // 1.09 ms at 2^24, 1.26 vs 2.12 at 2^25, ef44 2.92 vs 4.61 at 2^25; at 2^23
-  // 0.66 vs 0.57 ms and below it the 2^13-vertex bins are too few to fill the
-  // chip)
-  if (layout == kLayoutAuto && seg_log2 == 0 && kernel == 0 && graph->V >= (1u << 22) &&
-      ((uint64_t)graph->V + kPbSize - 1) / kPbSize <= kPbMaxBins && graph->E > 0)
-    layout = graph->V >= (1u << 24) && graph->E < 0xFFFFFFFFull ? kLayoutPairs : kLayoutBlocked;
+  // and over (source, bin) pairs from 2^24, and on skewed graphs -- a hub of
+  // 16 times the average out-degree, the mark of few pairs per edge -- from
+  // 3 * 2^22 edges on 2^18 vertices (twenty sweeps, ms, against the better of
+  // the two above: R-MAT 18 x 64 1.09 vs 1.10, 20 x 16 1.27 vs 1.46, 21 x 8 1.32 vs
+  // 1.70, 21 x 16 1.59 vs 2.95, 22 x 8 1.87 vs 3.26, 22 x 16 3.1 vs 6.9, 23 x 16
+  // 5.9 vs 11.3; fewer edges: 20 x 8 1.01 vs 0.73; without hubs, 2^22 vertices
+  // and uniform edges x 4 / x 16, 3.5 vs 1.8 and 6.9 vs 6.0)
+  const bool automatic = layout == kLayoutAuto && seg_log2 == 0 && kernel == 0 && graph->E > 0 &&
+                         ((uint64_t)graph->V + kPbSize - 1) / kPbSize <= kPbMaxBins;
+  if (automatic && graph->E < 0xFFFFFFFFull) {
+    const uint64_t avg = (graph->E + graph->V - 1) / graph->V;
+    const bool skewed = graph->max_outdeg >= 16 * avg;
+    if (graph->V >= (1u << 24)) layout = kLayoutPairs;
+    else if (skewed && graph->V >= (1u << 18) && graph->E >= 3ull << 22) {
+      PrPlan* p = new PrPlan();
+      const int st = build_pairs(graph, p, s);
+      if (st == CG_OK) {
+        *plan = p;
+        return CG_OK;
+      }
+      delete p;
+      // building the pairs takes the most memory: the others may still fit
+      if (st != CG_ERR_OOM) return st;
+      (void)hipGetLastError();
+    }
+  }
+  if (automatic && layout == kLayoutAuto && graph->V >= (1u << 22)) layout = kLayoutBlocked;
   if (layout == kLayoutPairs) {
     PrPlan* p = new PrPlan();
     const int st = build_pairs(graph, p, s);

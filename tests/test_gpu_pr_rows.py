@@ -72,3 +72,22 @@ def test_pair_groups(oracle):
             assert l1 <= 1e-6, (V, iters, l1)
         g.close()
 
+
+def test_automatic_layout(oracle):
+    """Pairs on skewed graphs from 3 * 2^22 edges; fewer edges, no hubs: the pull."""
+    m = 3 << 22
+    rng = np.random.default_rng(4)
+    V = 1 << 18
+    for skew, e_n, layout in ((2.5, m + 600000, 5), (2.5, m - 600000, 2), (1, m + 600000, 2)):
+        src = (V * rng.random(e_n) ** skew).astype(np.uint32)
+        dst = rng.integers(0, V, e_n).astype(np.uint32)
+        if skew > 1:
+            src[:20000] = 7
+        g = cg.Graph.from_edges(V, src, dst, None)
+        og = oracle.csr_build(V, src, dst)
+        e = cg.Engine(g, PR)
+        r, st = e.run()
+        e.close()
+        assert st["pr_layout"] == layout, (skew, e_n, st["pr_layout"])
+        assert float(np.abs(r.astype(np.float64) - oracle.pagerank64(og, 20, 0.85)).sum()) <= 1e-6
+        g.close()
