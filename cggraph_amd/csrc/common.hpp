@@ -16,6 +16,8 @@
 
 namespace cg {
 
+class HostStage;
+
 // Per-thread last error (cg_last_error).
 int set_error(int code, const char* fmt, ...) __attribute__((format(printf, 2, 3)));
 const char* last_error();
@@ -153,6 +155,7 @@ struct cg_graph {
   // batched queries: a copy renumbered by descending out-degree, built on
   // first use when the graph is large and skewed (vertex batch_new_of[v] of
   // the copy is the caller's v)
+  std::unique_ptr<cg::HostStage, void (*)(cg::HostStage*)> batch_stage{nullptr, nullptr};  // the batch's results (batch.hip)
   bool batch_relabel_done = false;
   std::unique_ptr<cg_graph> batch_rg;
   cg::DevBuf<uint32_t> batch_new_of;

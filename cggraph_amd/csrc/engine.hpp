@@ -9,6 +9,7 @@
 #include "cluster.hpp"
 #include "host_team.hpp"
 #include "kernels.hpp"
+#include "stage.hpp"
 #include "sched.hpp"
 
 struct cg_engine {
@@ -27,6 +28,7 @@ struct cg_engine {
   bool host_only = false;
 
   // values (uint32 for BFS/SSSP/CC, float for PR) and frontier state
+  cg::HostStage stage;  // results copied to the host
   cg::DevBuf<uint32_t> val;
   cg::DevBuf<uint32_t> xval;  // SSSP / CC fused pipeline: DevGraph::xval
   cg::DevBuf<uint64_t> bm[2];

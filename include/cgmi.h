@@ -310,8 +310,9 @@ int cg_graph_device_csr(const cg_graph* g, const uint64_t** offsets, const uint3
  * a HIP graph.  All three run at once.  stats: ms over all, iterations = the
  * largest level count, expand_launches = graph replays and cluster launches,
  * heavy_iterations = queries run on engines, edges_traversed =
- * the TEPS numerator over all queries.  mode 1: one query per engine launch
- * (the comparison path). */
+ * the TEPS numerator over all queries.  Values are copied out as queries end;
+ * after an error the buffers' contents are undefined.  mode 1: one query per
+ * engine launch (the comparison path). */
 int cg_batch_run(cg_graph* const* graphs, const int* algorithms, const uint32_t* roots, int nq,
                  uint32_t* const* outs, int mode, const cg_options* opt, cg_run_stats* stats);
 /* The same batched run over engine handles: query i is engine i's algorithm
