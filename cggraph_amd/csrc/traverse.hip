@@ -340,6 +340,7 @@ __global__ __launch_bounds__(kBlock) void k_init_traverse(TraverseInit a) {
         else if (j == offsetof(DevStats, n_chunk) / 4) x = f_chunk;
         else if (j == offsetof(DevStats, choice) / 4) x = f_pull;
         else if (j == offsetof(DevStats, chunk_edges) / 4) x = f_ce;
+        else if (j == offsetof(DevStats, min_val) / 4) x = 1;  // depth of what step 1 finds
       }
     }
     reinterpret_cast<uint32_t*>(a.st)[i] = x;
@@ -1749,6 +1750,7 @@ __global__ __launch_bounds__(NB) void k_bfs_front(const uint64_t* __restrict__ i
       for (int j = 0; j < 3; ++j) cnt_cur[k * kBfsCntStride + j] = 0;
     st->choice = pull ? 1 : 0;
     st->chunk_edges = ce;
+    st->min_val = w.iter;  // depth of what the step finds
     st_next->n_small = 0;
     st_next->n_med = 0;
     st_next->n_chunk = 0;
@@ -1774,6 +1776,11 @@ __global__ __launch_bounds__(NB) void k_bfs_front(const uint64_t* __restrict__ i
                         HubDefer{0, 1}, true, a);  // nothing dropped without values: `in` is only read
 }
 
+// in-edges a lane looks at together in a bottom-up BFS step
+// (R-MAT s24, edge factor 16: 1 / 2 / 3 / 4 517 / 512 / 509 / 525 us; s22 235 /
+// 233 / 230 / 222; s18 102 / 106 / 100 / 102)
+constexpr int kPullEdges = 3;
+
 template <bool EXACT>
 __global__ __launch_bounds__(kBlock) void k_bfs_step(DevGraph g, uint32_t* __restrict__ val,
                                                      const uint64_t* __restrict__ in, uint64_t* __restrict__ out,
@@ -1786,23 +1793,30 @@ __global__ __launch_bounds__(kBlock) void k_bfs_step(DevGraph g, uint32_t* __res
   if (st->choice == 1) {
     const uint64_t words = ((uint64_t)g.V + 63) / 64;
     const uint64_t nwaves = (uint64_t)gridDim.x * kWavesPerBlock;
+    const uint32_t depth = st->min_val;  // not from the parents' values: a line each (s24 547 -> 517 us)
     for (uint64_t w = (uint64_t)blockIdx.x * kWavesPerBlock + wave_id(); w < words; w += nwaves) {
       const uint64_t v = w * 64 + lane_id();
       bool found = false;
       if (v < g.V && val[v] == kUnreached) {
         const uint64_t s = g.in_off[v], e = g.in_off[v + 1];
-        for (uint64_t k = s; k < e; ++k) {
-          const uint32_t u = g.in_src[k];
-          if ((in[u >> 6] >> (u & 63)) & 1ull) {
-            val[v] = val[u] + 1;
-            found = true;
-            break;
-          }
+        for (uint64_t k = s; k < e && !found; k += kPullEdges) {
+          uint32_t x[kPullEdges];
+          uint64_t b[kPullEdges];
+#pragma unroll
+          for (int j = 0; j < kPullEdges; ++j) x[j] = g.in_src[k + j < e ? k + j : k];
+#pragma unroll
+          for (int j = 0; j < kPullEdges; ++j) b[j] = in[x[j] >> 6] >> (x[j] & 63);
+#pragma unroll
+          for (int j = 0; j < kPullEdges; ++j)
+            found |= (b[j] & 1ull) != 0;
         }
       }
       const uint64_t mask = __ballot(found);
       if (lane_id() == 0) out[w] = mask;
-      if (found) fv.first((uint32_t)v);
+      if (found) {
+        val[v] = depth;
+        fv.first((uint32_t)v);
+      }
     }
   } else {
     const uint32_t ce = st->chunk_edges ? st->chunk_edges : chunk_edges;
