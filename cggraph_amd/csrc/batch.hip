@@ -33,7 +33,7 @@
 // 20 us.  Level clusters (cluster.hpp) run them root to end, one launch for
 // all, beside the engines and the levels.  52 queries, four on each of R-MAT
 // s14-s22 and lattices of 256^2-2048^2: 126 -> 71 ms, the cluster launch 41
-// ms of it; with every query of the 512-query set off the engines 328 -> 215
+// ms of it (54.5 with the results copied while engines run); with every query of the 512-query set off the engines 328 -> 215
 // ms; with the s18-s22 queries on engines that set is bound by the engine
 // thread and stays at 237 ms.
 //

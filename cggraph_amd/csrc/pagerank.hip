@@ -10,7 +10,9 @@
 // Four layouts, chosen once per graph (the first three pull over the
 // in-edges, the fourth pushes through destination bins):
 //  plain       one sweep over the transposed graph per iteration, in blocks of
-//              consecutive rows staged through LDS (row blocks, below).
+//              consecutive rows staged through LDS (row blocks, below), or
+//              with rows tiered by in-degree: one lane / one wavefront per row,
+//              rows of 8192+ in-edges cut into 8192-edge chunks.
 //  relabelled  the same sweep over a copy of the CSC whose vertex ids are
 //              renumbered by descending out-degree (ties by id).  On skewed
 //              graphs a small prefix of the ids then carries most edges'
@@ -65,7 +67,8 @@ struct PrPlan {
     DevBuf<uint32_t> chunk_of;             // long row of each chunk
     DevBuf<double> partial;
   } rows;
-  // two-band sweep: tiers over the rows of the CSC in use, one set per pass
+  // row tiers over the CSC in use (one set per pass; the two-band sweep has
+  // two passes)
   struct Tiers {
     uint32_t n_med = 0, n_high = 0;
     DevBuf<uint32_t> med, high;
@@ -172,14 +175,15 @@ __device__ __forceinline__ void finish(uint32_t v, float sum, float base, float 
   contrib[v] = d ? r / (float)d : 0.0f;
 }
 
-// Row v's in-edges swept by pass P of the two-band sweep: 1 the sources below
-// the band boundary (a prefix, rows being sorted), 2 the rest.
+// Row v's in-edges swept by pass P: 0 the whole row; in the two-band sweep,
+// 1 the sources below the band boundary (a prefix, rows being sorted) and 2
+// the rest.
 template <int P>
 __device__ __forceinline__ void row_range(const Csc& g, uint32_t v, uint64_t& s, uint64_t& e) {
   s = g.off[v];
   e = g.off[v + 1];
   if constexpr (P == 1) e = s + g.hot[v];
-  else s += g.hot[v];
+  else if constexpr (P == 2) s += g.hot[v];
 }
 
 // Pass 1 keeps the partial sum; pass 2 adds the rest to it, so every row is
@@ -189,7 +193,8 @@ __device__ __forceinline__ void emit(const Csc& g, uint32_t v, float sum, float 
                                      float* __restrict__ part, float* __restrict__ rank,
                                      float* __restrict__ contrib) {
   if constexpr (P == 1) part[v] = sum;
-  else finish(v, part[v] + sum, base, damping, g.deg, rank, contrib);
+  else if constexpr (P == 2) finish(v, part[v] + sum, base, damping, g.deg, rank, contrib);
+  else finish(v, sum, base, damping, g.deg, rank, contrib);
 }
 
 // Rows with fewer than kMed in-edges in this pass: one lane per row, sources
@@ -925,6 +930,19 @@ int build_tiers(const Csc& g, PrPlan::Tiers& t, hipStream_t s) {
   CG_HIP(hipMemcpyAsync(t.row_chunk.p, first.data(), first.size() * 4, hipMemcpyHostToDevice, s));
   CG_HIP(hipStreamSynchronize(s));
   return CG_OK;
+}
+
+// Row blocks instead of row tiers: while the sources stay in the Infinity
+// Cache (256 MB) between sweeps.  Past it a block's fetch waits for HBM before
+// its gathers start, and lanes of one row each gather closer together (twenty
+// sweeps, blocks vs tiers, ms: R-MAT 20 x 32 2.5 vs 2.7, 21 x 16 3.0 vs 3.3, 22 x 8
+// 3.3 vs 4.4, 21 x 32 8.8 vs 6.5, 22 x 16 10.3 vs 7.7, 24 x 16 38.8 vs 34.2).  Not
+// on rows of a few neighbours in the caller's order, whose sources are
+// coalesced a lane per row too (lattice of 2048^2 0.82 vs 0.76, renumbered 0.92
+// vs 1.05).
+bool row_blocks_fit(uint32_t kernel, int layout, uint32_t V, uint64_t E) {
+  if (kernel == 1) return false;  // the tiers asked for
+  return E < 3ull << 24 && !(layout == kLayoutPlain && V > (1u << 16) && E < 4ull * V);
 }
 
 // Row blocks and the chunks of the long rows over a CSC.
@@ -2076,11 +2094,15 @@ int pr_plan_create(cg_graph* graph, uint32_t layout, uint32_t seg_log2, uint32_t
     } else if (kernel == 2) {
       st = build_tiles(p->r_off.p, g.V, E, p, s);
     } else {
-      st = build_rows(p->r_off.p, g.V, E, p->rows, s);
+      const Csc csc{p->r_off.p, p->r_src.p, p->deg.p, g.V, nullptr};
+      st = row_blocks_fit(kernel, kLayoutRelabel, g.V, E) ? build_rows(p->r_off.p, g.V, E, p->rows, s)
+                                                          : build_tiers<0>(csc, p->tiers[0], s);
     }
   } else if (st == CG_OK && p->layout == kLayoutPlain) {
+    const Csc csc{g.in_off, g.in_src, p->deg.p, g.V, nullptr};
     if (kernel == 2) st = build_tiles(g.in_off, g.V, E, p, s);
-    else st = build_rows(g.in_off, g.V, E, p->rows, s);
+    else if (row_blocks_fit(kernel, kLayoutPlain, g.V, E)) st = build_rows(g.in_off, g.V, E, p->rows, s);
+    else st = build_tiers<0>(csc, p->tiers[0], s);
   }
   if (st != CG_OK) {
     delete p;
@@ -2185,6 +2207,8 @@ int pr_run(const DevGraph& g, PrPlan* plan, int iters, float damping, float* ran
     } else if (plan->banded) {
       launch_tiers<1>(csc, plan->tiers[0], vblocks, c_cur, base, damping, plan->part.p, r_nxt, c_nxt, s);
       launch_tiers<2>(csc, plan->tiers[1], vblocks, c_cur, base, damping, plan->part.p, r_nxt, c_nxt, s);
+    } else if (!plan->rows.n) {
+      launch_tiers<0>(csc, plan->tiers[0], vblocks, c_cur, base, damping, nullptr, r_nxt, c_nxt, s);
     } else {
       const PrPlan::RowBlocks& b = plan->rows;
       const RowView view{b.row.p,      b.row_chunk.p, b.long_row.p, b.chunk_of.p, b.chunk_lo.p,

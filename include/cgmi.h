@@ -139,10 +139,11 @@ typedef struct cg_options {
                                      ids): 0 automatic (at least 2^21 vertices for SSSP, 2^23
                                      for BFS, and the top 1/64 of vertices send at least half of
                                      the edges), 1 never, 2 always */
-  uint32_t pr_kernel;             /* PageRank sweep over layouts 1 and 2: 0 automatic (row blocks,
-                                     the fastest measured), 1 row blocks (about 1024 in-edges
-                                     of consecutive rows per workgroup, longer rows in chunks;
-                                     64-bit sums), 2 edge tiles
+  uint32_t pr_kernel;             /* PageRank sweep over layouts 1 and 2: 0 automatic (row blocks
+                                     below 3 * 2^24 edges -- about 1024 in-edges of consecutive
+                                     rows per workgroup, longer rows in chunks, 64-bit sums --
+                                     else row tiers), 1 row tiers (a lane / wavefront /
+                                     workgroup per row by in-degree), 2 edge tiles
                                      (2048 consecutive in-edges per workgroup, rows combined by a
                                      segmented scan), 3 two source bands (renumbered layout: the
                                      sources below 2^pr_segment_log2, default 2^19, first, whose

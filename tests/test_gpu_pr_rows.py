@@ -31,12 +31,12 @@ def graphs(oracle):
     yield "renumbered", oracle.rmat_graph(17, 9, seed=6, weights=None)
 
 
-@pytest.mark.parametrize("layout", [1, 2])
-def test_row_blocks(oracle, layout):
+@pytest.mark.parametrize("layout,kernel", [(1, 0), (2, 0), (1, 1), (2, 1)])
+def test_row_blocks(oracle, layout, kernel):
     for name, og in graphs(oracle):
         g = cg.Graph.from_csr(og.offsets, og.dest)
         for iters in (0, 1, 2, 20):
-            e = cg.Engine(g, PR, pr_layout=layout, pr_iterations=iters)
+            e = cg.Engine(g, PR, pr_layout=layout, pr_kernel=kernel, pr_iterations=iters)
             r1, _ = e.run()
             r2, _ = e.run()
             e.close()
