@@ -639,6 +639,7 @@ int cg_engine_create(const cg_graph* cg, int algorithm, int engine_type, int use
   }
   const uint64_t V = g->V;
   const uint64_t words = (V + 63) / 64 + 1;
+  if (!e->host_only) CG_TRY(e->stage.prepare(V * 4));
   if (algorithm == CG_PR) {
     CG_TRY(e->rank.ensure(V));
     CG_TRY(e->rank2.ensure(V));

@@ -21,6 +21,10 @@ class HostStage {
       if (s.ev) (void)hipEventDestroy(s.ev);
   }
 
+  // The first buffer for results of n bytes, so that the first one does not
+  // wait for a pinned allocation (about 40 us).
+  int prepare(size_t n) { return fill(slot_[0], n < kPiece ? n : kPiece); }
+
   // Queues a copy of n bytes behind the stream's work.  The bytes are in dst
   // once finish() has returned.
   int put(void* dst, const void* src, size_t n, hipStream_t s) {
@@ -37,8 +41,7 @@ class HostStage {
       const size_t m = n - o < kPiece ? n - o : kPiece;
       Slot& t = slot_[next_];
       CG_TRY(empty(t));
-      CG_TRY(t.buf.ensure(m));
-      if (!t.ev) CG_HIP(hipEventCreateWithFlags(&t.ev, hipEventDisableTiming));
+      CG_TRY(fill(t, m));
       CG_HIP(hipMemcpyAsync(t.buf.p, static_cast<const uint8_t*>(src) + o, m, hipMemcpyDeviceToHost, s));
       CG_HIP(hipEventRecord(t.ev, s));
       t.dst = static_cast<uint8_t*>(dst) + o;
@@ -74,6 +77,11 @@ class HostStage {
     void* dst = nullptr;
     size_t n = 0;
   };
+  static int fill(Slot& t, size_t n) {
+    CG_TRY(t.buf.ensure(n));
+    if (!t.ev) CG_HIP(hipEventCreateWithFlags(&t.ev, hipEventDisableTiming));
+    return CG_OK;
+  }
   int empty(Slot& t) {
     if (!t.n) return CG_OK;
     CG_HIP(hipEventSynchronize(t.ev));
