@@ -26,8 +26,10 @@ __device__ __forceinline__ T add_agent(T* p, T x) {
 constexpr unsigned long long kMask40 = (1ull << 40) - 1;
 // A level's report, the sum of its workgroups': arrivals (6 bits) | those that
 // ask for the wide pipeline (6) | those with a long queue (6) | vertices (23) |
-// out-edges (23).  A workgroup's share of the last two saturates, so that 32
-// of them fit; both are exact up to the edge limit of a level.
+// out-edges (23).  A workgroup's share of the last two saturates, so that the
+// fields hold kClusterMaxGroups of them: a level's sums are exact unless one
+// of them reaches kShareMax (a row that long counts as kShareMax) or a queue
+// had no room (stop), which is beyond the edge limit of a level.
 constexpr int kFieldN = 23, kFieldM = 23, kFieldCount = 6;
 constexpr uint32_t kShareMax = 1u << 17;
 static_assert(kClusterMaxGroups < (1u << kFieldCount), "arrivals field");
@@ -583,6 +585,26 @@ __device__ __forceinline__ void cluster_run(ClusterShared& S, const ClusterJob& 
     edges = ld_agent(&ctl->edges_done);
     verts = ld_agent(&ctl->verts_done);
   }
+  // The front kernel sizes its chunks by the out-edges of the frontier handed
+  // back, so it needs their number even where the report's saturates; the
+  // vertices are exact (one level's edges discovered them).  One pass over the
+  // bitmap; bits of vertices without edges add nothing.
+  unsigned long long front_m = V.m;
+  if constexpr (ALG == CG_BFS) {
+    if (wide && k != J.k0 && (V.stop || V.m >= kShareMax)) {  // uniform over the cluster
+      const uint64_t* const front = J.bm[(k - 1) & 1];
+      unsigned long long ms = 0;
+      for (uint64_t i = gt; i < J.words; i += nthreads)
+        for (uint64_t bits = ld_agent(front + i); bits; bits &= bits - 1) {
+          const uint64_t v = i * 64 + (uint64_t)__builtin_ctzll(bits);
+          ms += J.off[v + 1] - J.off[v];
+        }
+      ms = wave_sum_u64(ms);
+      if (lane == 0 && ms) (void)add_agent(&ctl->edges_done, ms);
+      barrier(L + 1, 0);
+      front_m = ld_agent(&ctl->edges_done);
+    }
+  }
   if (gw != 0) return;
   if (wide && lane == 0) {
     if constexpr (ALG == CG_BFS) {
@@ -594,11 +616,13 @@ __device__ __forceinline__ void cluster_run(ClusterShared& S, const ClusterJob& 
       r.m_explored += edges;
       if (prev_n) r.prev_active = prev_n;
       J.rs[c] = r;
-      unsigned long long* const bc = J.bfs_cnt + (size_t)c * kBfsCntWords;
-      for (int i = 0; i < kStripes; ++i)
-        for (int j = 0; j < 3; ++j) bc[i * kBfsCntStride + j] = 0;
-      bc[0] = V.n;
-      bc[1] = V.m;
+      if (k != J.k0) {  // a frontier handed back as it was taken over has its counts
+        unsigned long long* const bc = J.bfs_cnt + (size_t)c * kBfsCntWords;
+        for (int i = 0; i < kStripes; ++i)
+          for (int j = 0; j < 3; ++j) bc[i * kBfsCntStride + j] = 0;
+        bc[0] = V.n;
+        bc[1] = front_m;
+      }
     } else {
       J.rs->iter = k - 1;
       J.rs->pad = 0;
