@@ -725,7 +725,8 @@ int run_batched(cg_graph* const* graphs, const int* algs, const uint32_t* roots,
   hipStream_t s = nullptr;
   CG_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
   std::unique_ptr<std::remove_pointer<hipStream_t>::type, decltype(&hipStreamDestroy)> sguard(s, hipStreamDestroy);
-  // level clusters: values and two bitmaps per query, queues per cluster.  A
+  // level clusters: values and two bitmaps per query (a bucketed one has a
+  // third), queues per cluster.  A
   // few queries get 16 workgroups each, many get 4, so that more run at once;
   // half of the chip is left to the engines and the level loop.
   const uint32_t cgroups = nc <= 8 ? 16 : (nc <= 32 ? 8 : 4);
@@ -736,7 +737,7 @@ int run_batched(cg_graph* const* graphs, const int* algs, const uint32_t* roots,
   for (int k = 0; k < nc; ++k) {
     const uint64_t V = graphs[cq[k]]->V;
     cpre[k + 1] = cpre[k] + (V + 31) / 32 * 32;
-    wpre[k + 1] = wpre[k] + 2 * ((V + 63) / 64);
+    wpre[k + 1] = wpre[k] + (algs[cq[k]] == CG_SSSP && opt.sssp_delta ? 3 : 2) * ((V + 63) / 64);
   }
   // the level loop: values, stamps and two frontier queues per query
   std::vector<uint64_t> vpre(nb + 1, 0);

@@ -255,8 +255,8 @@ __device__ __forceinline__ void cluster_run(ClusterShared& S, const ClusterJob& 
   // fl.  An entry whose vertex has a smaller value by the time the list is
   // split is dropped there: the improvement queued the vertex again.
   auto far_at = [&](uint32_t fl, uint32_t i) { return J.far[fl & 1] + (size_t)id * kClusterFar + i; };
-  // Returns true where there is no room: the vertex then goes into the frontier
-  // that is handed back.
+  // Without room for it the vertex waits in the bitmap (BATCH), or the result
+  // is true: it then goes into the frontier that is handed back.
   auto push_far = [&](bool p, uint32_t v, uint32_t value, uint32_t fl) -> bool {
     const uint64_t pm = __ballot(p);
     if (!pm) return false;
@@ -275,6 +275,11 @@ __device__ __forceinline__ void cluster_run(ClusterShared& S, const ClusterJob& 
     const uint32_t pos = lane_value(base, 0) + (uint32_t)__popcll(pm & ((1ull << lane) - 1));
     if (p && pos < kClusterFar) st_agent(far_at(fl, pos), (unsigned long long)value << 32 | v);
     const bool full = p && pos >= kClusterFar;
+    if constexpr (BATCH) {
+      if (full) set_bit(J.wait, v);
+      if (__ballot(full) && lane == 0) st_agent(&ctl->far[fl % 3].over, 1u);
+      return false;
+    }
     if (full) stop = 1;
     return full;
   };
@@ -386,11 +391,14 @@ __device__ __forceinline__ void cluster_run(ClusterShared& S, const ClusterJob& 
       // (nothing is added to it in this level, so every wavefront reads the same)
       const uint32_t far_count = ld_agent(&ctl->far[F % 3].count), far_min = ld_agent(&ctl->far[F % 3].min_val);
       if (!far_count) break;
+      const uint32_t last_thr = thr;
+      const bool over = BATCH && ld_agent(&ctl->far[F % 3].over) != 0;
       const uint64_t nt = (uint64_t)far_min + J.delta;
       thr = nt > 0xFFFFFFFEull ? 0xFFFFFFFEu : (uint32_t)nt;
       if (gt == 0) {
         st_agent(&ctl->far[(F + 2) % 3].count, 0u);
         st_agent(&ctl->far[(F + 2) % 3].min_val, kClusterNone);
+        st_agent(&ctl->far[(F + 2) % 3].over, 0u);
       }
       const uint32_t own = S.far_cnt[F & 1] < kClusterFar ? S.far_cnt[F & 1] : kClusterFar;
       for (uint32_t b = wv * kWave; b < own; b += kClusterBlock) {  // wave-uniform
@@ -410,6 +418,53 @@ __device__ __forceinline__ void cluster_run(ClusterShared& S, const ClusterJob& 
         if (near) set_bit(bout, v);
         push(near, v, x, s, e - s, qp);
         if (push_far(valid && x >= thr, v, x, F + 1)) set_bit(bout, v);
+      }
+      if (over) {
+        // the bitmap of those without room: a value below the last threshold
+        // has improved since (and was queued), one that still waits keeps its
+        // bit and counts for the next split
+        const uint64_t places = (J.words + 7) / 8;
+        uint32_t stay_n = 0, stay_min = kClusterNone;  // per lane
+        for (uint64_t r = 0; r * 8 * nwaves < places; ++r) {  // uniform
+          const uint64_t i = ((r * 8 + lane / 8) * nwaves + wv * members + id) * 8 + lane % 8;
+          uint64_t bits = i < J.words ? ld_agent(J.wait + i) : 0ull, gone = 0;
+          while (__ballot(bits != 0)) {
+            bool near = false;
+            uint32_t v = 0, x = 0;
+            uint64_t s = 0, e = 0;
+            if (bits) {
+              const int j = __builtin_ctzll(bits);
+              bits &= bits - 1;
+              v = (uint32_t)(i * 64 + (uint64_t)j);
+              x = ld_agent(J.val + v);
+              if (x >= thr) {
+                ++stay_n;
+                stay_min = x < stay_min ? x : stay_min;
+              } else {
+                gone |= 1ull << j;
+                near = x >= last_thr;
+              }
+              if (near) {
+                s = J.off[v];
+                e = J.off[v + 1];
+                set_bit(bout, v);
+              }
+            }
+            push(near, v, x, s, e - s, qp);
+          }
+          // (bits that the lists' vertices set meanwhile stay)
+          if (gone)
+            (void)__hip_atomic_fetch_and(reinterpret_cast<unsigned long long*>(J.wait) + i, ~(unsigned long long)gone,
+                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        stay_n = wave_sum_u32(stay_n);
+        stay_min = wave_min_u32(stay_min);
+        if (lane == 0 && stay_n) {
+          ClusterFarState* const next = &ctl->far[(F + 1) % 3];
+          (void)add_agent(&next->count, stay_n);
+          (void)__hip_atomic_fetch_min(&next->min_val, stay_min, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          st_agent(&next->over, 1u);
+        }
       }
       __syncthreads();
       if (t == 0) S.far_cnt[F & 1] = 0;
@@ -697,6 +752,7 @@ __global__ __launch_bounds__(kClusterBlock) void k_cluster_batch(ClusterBatch b)
     J.threshold = Q.delta;
     J.ctl = ctl;
     J.batch_levels = b.levels;
+    J.wait = Q.bm + 2 * Q.words;
     if (Q.alg == CG_BFS) cluster_run<CG_BFS, uint32_t, true>(S, J);
     else cluster_run<CG_SSSP, uint32_t, true>(S, J);
   }
