@@ -540,6 +540,30 @@ static double batch_cluster_cost(const cg_graph* g, int alg) {
   return 20.0 + (double)g->E / 10000.0;
 }
 
+// Whether the levels of a query that a cluster could run are wide although the
+// rows are short: SSSP without buckets, whose frontier is every vertex that
+// improved last, up to a tenth of the graph.  The whole chip takes such a query
+// in a fraction of the time: an engine of the graph 33 / 95 / 18 / 7.4 ms (1000^2
+// and 2048^2 lattices, 160^3, 2^22 vertices of 16 uniform edges) where a cluster
+// takes 96 / 1552 / 120 / 75 alone, 181 / 2742 / 359 / 153 with nine at once.
+// Below 2^20 edges the two are alike (400^2: 7.5 and 7.2; two of four queries on
+// engines at 300^2 / 40^3 9.6 / 3.7 instead of 5.9 / 2.2).
+constexpr uint64_t kBatchWideEdges = 1u << 20;
+static bool batch_wide_on_cluster(const cg_graph* g, int alg, const cg_options& opt) {
+  return alg == CG_SSSP && !opt.sssp_delta && g->E >= kBatchWideEdges;
+}
+// How many of them, equal ones, run one after another before a cluster would
+// have ended: grows with the graph (2.0-2.9 at 1.3 to 3.6 M edges of a 2-D
+// lattice, 4.2-16 from 8 M; 2.6-8.6 in 3-D, 4-10 uniform; with nine at once
+// about twice that).  Where the caller keeps the batch off engines they join the
+// level loop, which takes about three times as long (43 / 312 / 64 / 53 ms).
+static double batch_wide_rate(const cg_graph* g, bool engines) {
+  const double r = std::min(std::max((double)g->E / 1.0e6, 2.0), 10.0);
+  return engines ? r : r / 3.0;
+}
+// Its time on an engine, in some unit (lattices: 18 ms at 600^2 vertices, 190 at 3000^2).
+static double batch_wide_cost(const cg_graph* g) { return std::pow((double)g->V, 0.75); }
+
 // The buffers a batch's results leave through: those kept with its first
 // graph, or some of its own while another batch uses them.  Copies under way
 // when the batch ends early are dropped.
@@ -689,6 +713,44 @@ int run_batched(cg_graph* const* graphs, const int* algs, const uint32_t* roots,
       bq.push_back(i);
     }
   }
+  std::stable_sort(cq.begin(), cq.end(), [&](int a, int b) {
+    return batch_cluster_cost(graphs[a], algs[a]) > batch_cluster_cost(graphs[b], algs[b]);
+  });
+  // of the wide ones, longest first, as many leave the clusters as end before
+  // those that stay
+  const bool others = !jobs.empty() || !bq.empty();  // queries that were never a cluster's
+  {
+    const bool engines = min_v != 0xFFFFFFFFu;
+    double busy = 0.0;
+    size_t kept = 0;
+    for (int i : cq) {
+      const double t = batch_wide_cost(graphs[i]);
+      bool stays = !batch_wide_on_cluster(graphs[i], algs[i], opt) ||
+                   busy + t > batch_wide_rate(graphs[i], engines) * t;
+      // a BFS alone may be wide too, and an engine is no slower if it is not
+      // (2^22 vertices of 16 uniform edges 11.5 ms on a cluster, 6.1 level by
+      // level, 0.5 on an engine; lattices of 160^3 13 / 9.5 / 6.3, 1000^2 7 / 18 / 6)
+      if (nq == 1 && algs[i] == CG_BFS && engines && graphs[i]->E >= kBatchWideEdges) stays = false;
+      if (!stays && engines) {
+        cg_engine* e = nullptr;
+        const int rc = batch_engine(graphs[i], algs[i], &e);
+        if (rc == CG_OK) {
+          jobs.push_back(EngineQuery{e, roots[i], nullptr});
+          jq.push_back(i);
+        } else if (rc == CG_ERR_OOM) {
+          clear_error();
+          stays = true;  // a cluster needs less
+        } else {
+          return rc;
+        }
+      } else if (!stays) {
+        bq.push_back(i);
+      }
+      if (stays) cq[kept++] = i;
+      else busy += t;
+    }
+    cq.resize(kept);
+  }
   uint64_t slot_v = 0;
   for (int i : jq) slot_v += graphs[i]->V;
   DevBuf<uint32_t> slots;
@@ -702,9 +764,6 @@ int run_batched(cg_graph* const* graphs, const int* algs, const uint32_t* roots,
     }
   }
   const int nb = (int)bq.size(), nc = (int)cq.size();
-  std::stable_sort(cq.begin(), cq.end(), [&](int a, int b) {
-    return batch_cluster_cost(graphs[a], algs[a]) > batch_cluster_cost(graphs[b], algs[b]);
-  });
   // the graph each batched query runs on, its root there, and the map back
   std::vector<cg_graph*> qgraph(nb);
   std::vector<uint32_t> qroot(nb);
@@ -728,9 +787,10 @@ int run_batched(cg_graph* const* graphs, const int* algs, const uint32_t* roots,
   // level clusters: values and two bitmaps per query (a bucketed one has a
   // third), queues per cluster.  A
   // few queries get 16 workgroups each, many get 4, so that more run at once;
-  // half of the chip is left to the engines and the level loop.
+  // half of the chip is left to the engines and the level loop (not to the wide
+  // queries that left the clusters, which are to end sooner anyway).
   const uint32_t cgroups = nc <= 8 ? 16 : (nc <= 32 ? 8 : 4);
-  const uint32_t clusters = std::min<uint32_t>((uint32_t)nc, (jobs.empty() && !nb ? 256u : 128u) / cgroups);
+  const uint32_t clusters = std::min<uint32_t>((uint32_t)nc, (others ? 128u : 256u) / cgroups);
   DevBuf<uint32_t> cval;
   DevBuf<uint64_t> cbm, cq_mem;
   std::vector<uint64_t> cpre(nc + 1, 0), wpre(nc + 1, 0);

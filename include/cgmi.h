@@ -186,7 +186,11 @@ typedef struct cg_options {
                                      schedule; SSSP defers hubs of out-degree >= 128 within
                                      max weight / 50 of the frontier's smallest), on a host thread
                                      of their own while the other queries advance level by
-                                     level; 0 = 2^18, 0xFFFFFFFF = every query batched.  The
+                                     level; 0 = 2^18, 0xFFFFFFFF = every query batched.  Of the
+                                     SSSP queries without sssp_delta on graphs of out-degrees
+                                     up to 64 and 2^20 edges or more, a few join the engines
+                                     whatever the size, as many as end before the rest (and a
+                                     BFS on such a graph that is the batch's only query).  The
                                      engines belong to the graph, so batches running at once
                                      from several threads take turns for their engine queries */
 } cg_options;
@@ -306,7 +310,9 @@ int cg_graph_device_csr(const cg_graph* g, const uint64_t** offsets, const uint3
  * graph from a host thread of their own; those on graphs of narrow frontiers
  * (largest out-degree at most 64) or of at most 2^18 edges run root to end in
  * one launch whose clusters of workgroups take a query each (batch_block,
- * batch_grid, batch_levels, batch_group and hub deferral do not apply there);
+ * batch_grid, batch_levels, batch_group and hub deferral do not apply there;
+ * a few of the SSSP queries without buckets, whose levels are wide, join the
+ * engines, see batch_engine_v);
  * the others advance level by level together, the per-level loop captured in
  * a HIP graph.  All three run at once.  stats: ms over all, iterations = the
  * largest level count, expand_launches = graph replays and cluster launches,

@@ -1,0 +1,62 @@
+"""SSSP queries without buckets on graphs of short rows: a batch gives as many
+to engines of their graphs (with engines off, to the level loop) as end before
+the clusters do with the rest.  Every route bit-exact against the oracle, alone
+and beside queries that stay, and the number that leave by the rule."""
+import numpy as np
+import pytest
+
+import cggraph_amd as cg
+from cggraph_amd import batch
+
+pytestmark = pytest.mark.gpu
+BFS, SSSP = 0, 1
+
+
+@pytest.fixture(scope="module")
+def graphs(oracle):
+    rng = np.random.default_rng(2)
+    uniform = oracle.csr_build(70_000, rng.integers(0, 70_000, 1_100_000).astype(np.uint32),
+                               rng.integers(0, 70_000, 1_100_000).astype(np.uint32))
+    uniform.weight = rng.integers(1, 70_000, uniform.E).astype(np.uint32)
+    ogs = [oracle.grid_graph(530, 0.1, seed=1),  # below 2^20 edges
+           oracle.grid_graph(560, 0.1, seed=1), uniform, oracle.rmat_graph(12, 16, seed=5, weights=(1, 1000))]
+    assert ogs[0].E < 1 << 20 < min(ogs[1].E, uniform.E) and np.diff(uniform.offsets.astype(np.int64)).max() <= 64
+    hs = [cg.Graph.from_csr(o.offsets, o.dest, o.weight) for o in ogs]
+    yield ogs, hs
+    for h in hs:
+        h.close()
+
+
+@pytest.mark.parametrize("which", [(1,), (2,), (0, 1, 2, 3), (2, 1)])
+@pytest.mark.parametrize("n", [1, 2, 3, 12])
+def test_routes(oracle, graphs, which, n):
+    ogs, hs = graphs
+    qs = [(k, a, (7919 * i + 13 * k) % ogs[k].V) for i in range(n) for k in which for a in (SSSP, BFS)]
+    refs = {q: (oracle.bfs if q[1] == BFS else oracle.sssp)(ogs[q[0]], q[2]) for q in set(qs)}
+    edges = sum(oracle.reached_edges(ogs[q[0]], refs[q]) for q in qs)
+    for opt in ({}, {"batch_engine_v": 0xFFFFFFFF}, {"sssp_delta": 2000}, {"batch_engine_v": 1}):
+        outs, st = batch.run_batch([hs[k] for k, _, _ in qs], [a for _, a, _ in qs], [r for _, _, r in qs], **opt)
+        for q, got in zip(qs, outs):
+            assert np.array_equal(got, refs[q]), (q, opt)
+        assert st["edges_traversed"] == edges
+        skewed = 2 * n * which.count(3) if opt.get("batch_engine_v") == 1 else 0
+        if "sssp_delta" in opt or opt.get("batch_engine_v") == 0xFFFFFFFF:
+            leave = 0
+        else:  # longest first while the sum stays within twice the next one's time (below 2 M edges)
+            busy, leave = 0.0, 0
+            order = sorted((k for k, a, _ in qs if a == SSSP and k in (1, 2)), key=lambda k: -ogs[k].V)
+            for k in order:
+                t = ogs[k].V ** 0.75
+                if busy + t <= 2 * t:
+                    busy, leave = busy + t, leave + 1
+        assert st["heavy_iterations"] == leave + skewed, (opt, leave, skewed)
+
+
+def test_lone_bfs(oracle, graphs):
+    ogs, hs = graphs
+    for k, engine in ((0, 0), (1, 1), (2, 1)):
+        for opt in ({}, {"batch_engine_v": 0xFFFFFFFF}):
+            for r in (3, ogs[k].V - 1):
+                (got,), st = batch.run_batch([hs[k]], [BFS], [r], **opt)
+                assert np.array_equal(got, oracle.bfs(ogs[k], r)), (k, r, opt)
+                assert st["heavy_iterations"] == (0 if opt else engine)
