@@ -548,9 +548,16 @@ static double batch_cluster_cost(const cg_graph* g, int alg) {
 // takes 96 / 1552 / 120 / 75 alone, 181 / 2742 / 359 / 153 with nine at once.
 // Below 2^20 edges the two are alike (400^2: 7.5 and 7.2; two of four queries on
 // engines at 300^2 / 40^3 9.6 / 3.7 instead of 5.9 / 2.2).
+// With unit weights its frontiers are BFS's and it stays (nine queries on 1000^2
+// 9 ms, 22 with three of them on an engine).
 constexpr uint64_t kBatchWideEdges = 1u << 20;
-static bool batch_wide_on_cluster(const cg_graph* g, int alg, const cg_options& opt) {
-  return alg == CG_SSSP && !opt.sssp_delta && g->E >= kBatchWideEdges;
+static int batch_wide_on_cluster(cg_graph* g, int alg, const cg_options& opt, bool* wide) {
+  *wide = false;
+  if (alg != CG_SSSP || opt.sssp_delta || g->E < kBatchWideEdges) return CG_OK;
+  std::lock_guard<std::mutex> lock(batch_relabel_mu);
+  CG_TRY(ensure_narrow_weights(g, nullptr));  // finds the largest weight
+  *wide = g->max_w > 1;
+  return CG_OK;
 }
 // How many of them, equal ones, run one after another before a cluster would
 // have ended: grows with the graph (2.0-2.9 at 1.3 to 3.6 M edges of a 2-D
@@ -725,24 +732,24 @@ int run_batched(cg_graph* const* graphs, const int* algs, const uint32_t* roots,
     size_t kept = 0;
     for (int i : cq) {
       const double t = batch_wide_cost(graphs[i]);
-      bool stays = !batch_wide_on_cluster(graphs[i], algs[i], opt) ||
-                   busy + t > batch_wide_rate(graphs[i], engines) * t;
+      bool wide = false;
+      int rc = batch_wide_on_cluster(graphs[i], algs[i], opt, &wide);
+      bool stays = !wide || busy + t > batch_wide_rate(graphs[i], engines) * t;
       // a BFS alone may be wide too, and an engine is no slower if it is not
       // (2^22 vertices of 16 uniform edges 11.5 ms on a cluster, 6.1 level by
       // level, 0.5 on an engine; lattices of 160^3 13 / 9.5 / 6.3, 1000^2 7 / 18 / 6)
       if (nq == 1 && algs[i] == CG_BFS && engines && graphs[i]->E >= kBatchWideEdges) stays = false;
+      cg_engine* e = nullptr;
+      if (rc == CG_OK && !stays && engines) rc = batch_engine(graphs[i], algs[i], &e);
+      if (rc == CG_ERR_OOM) {  // a cluster needs less
+        clear_error();
+        stays = true;
+      } else if (rc != CG_OK) {
+        return rc;
+      }
       if (!stays && engines) {
-        cg_engine* e = nullptr;
-        const int rc = batch_engine(graphs[i], algs[i], &e);
-        if (rc == CG_OK) {
-          jobs.push_back(EngineQuery{e, roots[i], nullptr});
-          jq.push_back(i);
-        } else if (rc == CG_ERR_OOM) {
-          clear_error();
-          stays = true;  // a cluster needs less
-        } else {
-          return rc;
-        }
+        jobs.push_back(EngineQuery{e, roots[i], nullptr});
+        jq.push_back(i);
       } else if (!stays) {
         bq.push_back(i);
       }

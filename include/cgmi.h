@@ -187,9 +187,9 @@ typedef struct cg_options {
                                      max weight / 50 of the frontier's smallest), on a host thread
                                      of their own while the other queries advance level by
                                      level; 0 = 2^18, 0xFFFFFFFF = every query batched.  Of the
-                                     SSSP queries without sssp_delta on graphs of out-degrees
-                                     up to 64 and 2^20 edges or more, a few join the engines
-                                     whatever the size, as many as end before the rest (and a
+                                     SSSP queries without sssp_delta on graphs of out-degrees up
+                                     to 64, weights above 1 and 2^20 edges or more, a few join
+                                     the engines, as many as end before the rest (and a
                                      BFS on such a graph that is the batch's only query).  The
                                      engines belong to the graph, so batches running at once
                                      from several threads take turns for their engine queries */

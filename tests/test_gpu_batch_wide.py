@@ -60,3 +60,13 @@ def test_lone_bfs(oracle, graphs):
                 (got,), st = batch.run_batch([hs[k]], [BFS], [r], **opt)
                 assert np.array_equal(got, oracle.bfs(ogs[k], r)), (k, r, opt)
                 assert st["heavy_iterations"] == (0 if opt else engine)
+
+
+def test_unit_weights_stay(oracle, graphs):
+    og = graphs[0][1]
+    h = cg.Graph.from_csr(og.offsets, og.dest, np.ones(og.E, np.uint32))
+    outs, st = batch.run_batch([h] * 3, [SSSP] * 3, [0, 5, og.V - 1])
+    assert st["heavy_iterations"] == 0
+    for r, got in zip([0, 5, og.V - 1], outs):
+        assert np.array_equal(got, oracle.bfs(og, r))
+    h.close()
