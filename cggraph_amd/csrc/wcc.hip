@@ -62,20 +62,41 @@ __device__ void link(uint32_t u, uint32_t v, uint32_t* __restrict__ parent) {
   }
 }
 
-// The root above v, given its parent and grandparent; every step is stored,
-// so the climbs of a long chain's vertices shorten each other.
-__device__ __forceinline__ uint32_t climb(uint32_t v, uint32_t p, uint32_t gp, uint32_t* __restrict__ parent) {
-  while (p != gp) {
-    __hip_atomic_store(parent + v, gp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    p = gp;
-    gp = ld_relaxed(parent + p);
+// Climbs from the lane's N vertices base + k * stride (those below V), given
+// their parents p and grandparents gp, to their roots p; every step is stored,
+// so the climbs of a long chain's vertices shorten each other.  The N climb
+// together: one after the other, those that wait leave their part of the chain
+// one step long for every climb above it (paths of 0.1 / 1 / 4 M vertices 331 /
+// 420 / 910 us per query, together 68 / 100 / 240; lattices of 300^2 / 1000^2 /
+// 2048^2 101 / 203 / 550, together 90 / 168 / 465).
+template <int N>
+__device__ __forceinline__ void climb(uint64_t base, uint32_t stride, uint32_t V, uint32_t (&p)[N], uint32_t (&gp)[N],
+                                      uint32_t* __restrict__ parent) {
+  bool more = true;
+  while (more) {
+    more = false;
+    bool moved[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      moved[k] = p[k] != gp[k] && base + k * stride < V;
+      if (moved[k]) {
+        __hip_atomic_store(parent + base + k * stride, gp[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        p[k] = gp[k];
+        more = true;
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+      if (moved[k]) gp[k] = ld_relaxed(parent + p[k]);
   }
-  return p;
 }
 
 // Round 0: parent[v] = min(v, first neighbour).  Bound by one line per row
 // (off is streamed); kIlp rows per lane keep that many in flight.
 constexpr int kIlp = 4;
+// and where chains are climbed (lattices of 100^2 / 300^2 / 1000^2 / 2048^2, us per
+// query with 4: 69 / 94 / 168 / 453, 2: 64 / 90 / 168 / 465, 1: 62 / 90 / 175 / 518)
+constexpr int kChainIlp = 2;
 
 __global__ __launch_bounds__(kBlock) void k_first(DevGraph g, uint32_t* __restrict__ parent) {
   const uint64_t base = blockIdx.x * (uint64_t)(kBlock * kIlp) + threadIdx.x;
@@ -113,19 +134,18 @@ __global__ __launch_bounds__(kBlock) void k_link_round(DevGraph g, uint32_t r, c
 }
 
 // plan: only if that many rounds were linked (NULL: always).
+template <int ILP>
 __global__ __launch_bounds__(kBlock) void k_compress(uint32_t V, uint32_t* __restrict__ parent,
                                                      const WccPlan* __restrict__ plan, uint32_t rounds) {
   if (plan && plan->rounds != rounds) return;
-  for (uint64_t base = blockIdx.x * (uint64_t)(kBlock * kIlp) + threadIdx.x; base < V;
-       base += (uint64_t)gridDim.x * (kBlock * kIlp)) {
-    uint32_t p[kIlp], gp[kIlp];
+  for (uint64_t base = blockIdx.x * (uint64_t)(kBlock * ILP) + threadIdx.x; base < V;
+       base += (uint64_t)gridDim.x * (kBlock * ILP)) {
+    uint32_t p[ILP], gp[ILP];
 #pragma unroll
-    for (int k = 0; k < kIlp; ++k) p[k] = base + k * kBlock < V ? ld_relaxed(parent + base + k * kBlock) : 0u;
+    for (int k = 0; k < ILP; ++k) p[k] = base + k * kBlock < V ? ld_relaxed(parent + base + k * kBlock) : 0u;
 #pragma unroll
-    for (int k = 0; k < kIlp; ++k) gp[k] = ld_relaxed(parent + p[k]);
-#pragma unroll
-    for (int k = 0; k < kIlp; ++k)
-      if (base + k * kBlock < V) (void)climb((uint32_t)(base + k * kBlock), p[k], gp[k], parent);
+    for (int k = 0; k < ILP; ++k) gp[k] = ld_relaxed(parent + p[k]);
+    climb<ILP>(base, kBlock, V, p, gp, parent);
   }
 }
 
@@ -212,9 +232,7 @@ __global__ __launch_bounds__(kBlock) void k_link_rest(DevGraph g, const WccPlan*
   for (int k = 0; k < kIlp; ++k) p[k] = base + k * 64 < g.V ? ld_relaxed(parent + base + k * 64) : skip;
 #pragma unroll
   for (int k = 0; k < kIlp; ++k) gp[k] = ld_relaxed(parent + p[k]);
-#pragma unroll
-  for (int k = 0; k < kIlp; ++k)
-    if (base + k * 64 < g.V) p[k] = climb((uint32_t)(base + k * 64), p[k], gp[k], parent);
+  climb<kIlp>(base, 64, g.V, p, gp, parent);
 #pragma unroll 1
   for (int k = 0; k < kIlp; ++k) {
     const uint64_t v = base + k * 64;
@@ -246,15 +264,16 @@ int wcc_hooking(const DevGraph& g, uint32_t* parent, void* workspace, hipStream_
   WccPlan* const plan = static_cast<WccPlan*>(workspace);
   constexpr uint64_t kSeed = 0x5EEDull;
   const dim3 block(kBlock), rows((unsigned)(((uint64_t)V + kBlock * kIlp - 1) / (kBlock * kIlp)));
-  const dim3 capped(std::min(rows.x, 2048u));  // strides; most often it returns at once
+  // strides; most often these return at once
+  const dim3 capped(std::min(rows.x, 2048u)), chains(std::min(rows.x * (kIlp / kChainIlp), 2048u));
   hipLaunchKernelGGL(k_first, rows, block, 0, s, g, parent);
   hipLaunchKernelGGL(k_sample, dim3(1), dim3(kSamples), 0, s, g, parent, kSeed, 1u, plan);
-  hipLaunchKernelGGL(k_compress, capped, block, 0, s, V, parent, plan, 2u);
+  hipLaunchKernelGGL(k_compress<kChainIlp>, chains, block, 0, s, V, parent, plan, 2u);
   hipLaunchKernelGGL(k_link_round, capped, block, 0, s, g, 1u, plan, parent);
-  hipLaunchKernelGGL(k_compress, capped, block, 0, s, V, parent, plan, 2u);
+  hipLaunchKernelGGL(k_compress<kChainIlp>, chains, block, 0, s, V, parent, plan, 2u);
   hipLaunchKernelGGL(k_sample, dim3(1), dim3(kSamples), 0, s, g, parent, kSeed, 2u, plan);
   hipLaunchKernelGGL(k_link_rest, rows, block, 0, s, g, plan, parent);
-  hipLaunchKernelGGL(k_compress, rows, block, 0, s, V, parent, (const WccPlan*)nullptr, 0u);
+  hipLaunchKernelGGL(k_compress<kIlp>, rows, block, 0, s, V, parent, (const WccPlan*)nullptr, 0u);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return set_error(CG_ERR_HIP, "WCC kernels: %s", hipGetErrorString(e));
   return CG_OK;
