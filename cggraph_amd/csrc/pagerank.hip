@@ -1848,7 +1848,46 @@ int pb_tiles(PrPlan* p, const std::vector<uint64_t>& hb, const std::vector<uint6
   return CG_OK;
 }
 
-int build_pairs(cg_graph* graph, PrPlan* p, hipStream_t s) {
+// Whether pairs beat the blocked layout from 2^22 vertices on (below, the other
+// one is the renumbered pull, which they always beat).  A pair for every edge
+// costs what an edge costs there and the gather's locality on top; the line is
+// at 0.85 pairs an edge (twenty sweeps, pairs and blocked, ms, at 2^22 vertices
+// and 16.8 M edges: 0.40 1.41 / 3.7, 0.75 1.58 / 3.2, 0.94 2.45 / 1.75, 0.996 with
+// one hub 2.71 / 1.82; 67 M: 0.26 3.1 / 7.0, 0.82 5.4 / 7.1, 0.89 6.5 / 5.7, 0.985
+// 6.9 / 5.9).  But where a bin of the caller's destinations has kPairHotBin times
+// its share, the blocked layout waits for it (4 times: 0.89 1.9 / 2.9, 8: 0.93
+// 2.0 / 2.6, 22: 0.98 2.2 / 3.2), and where the top 1/64 of vertices send little no source has
+// many edges in a bin (the one hub 0.04, R-MAT a = 0.35 0.07: 2.3 / 1.9).
+constexpr double kPairShare = 0.1, kPairRate = 0.85;
+constexpr uint32_t kPairHotBin = 3;
+
+__global__ __launch_bounds__(kBlock) void k_bin_counts(const uint32_t* __restrict__ dst, uint64_t E, uint32_t nb,
+                                                       uint32_t* __restrict__ cnt) {
+  __shared__ uint32_t lc[kPbMaxBins];
+  for (uint32_t b = threadIdx.x; b < nb; b += kBlock) lc[b] = 0;
+  __syncthreads();
+  for (uint64_t e = blockIdx.x * (uint64_t)kBlock + threadIdx.x; e < E; e += (uint64_t)gridDim.x * kBlock)
+    atomicAdd(&lc[dst[e] >> kPbShift], 1u);
+  __syncthreads();
+  for (uint32_t b = threadIdx.x; b < nb; b += kBlock)
+    if (lc[b]) atomicAdd(&cnt[b], lc[b]);
+}
+
+int hot_bin(const cg_graph* g, uint32_t nb, bool* hot, hipStream_t s) {
+  DevBuf<uint32_t> cnt;
+  CG_TRY(cnt.ensure(nb));
+  CG_HIP(hipMemsetAsync(cnt.p, 0, nb * sizeof(uint32_t), s));
+  hipLaunchKernelGGL(k_bin_counts, dim3(1024), dim3(kBlock), 0, s, g->d_dst.p, g->E, nb, cnt.p);
+  PR_LAUNCH_OK();
+  std::vector<uint32_t> h(nb);
+  CG_HIP(hipMemcpyAsync(h.data(), cnt.p, nb * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+  CG_HIP(hipStreamSynchronize(s));
+  *hot = (uint64_t)*std::max_element(h.begin(), h.end()) * nb >= kPairHotBin * g->E;
+  return CG_OK;
+}
+
+// few not NULL: stops where pairs would not beat the blocked layout (*few false).
+int build_pairs(cg_graph* graph, PrPlan* p, hipStream_t s, bool* few = nullptr) {
   const uint32_t V = graph->V;
   const uint64_t E = graph->E;
   const uint32_t nb = (uint32_t)(((uint64_t)V + kPbSize - 1) >> kPbShift);
@@ -1861,7 +1900,12 @@ int build_pairs(cg_graph* graph, PrPlan* p, hipStream_t s) {
   cg_graph rg;
   {
     DevBuf<uint32_t> new_of;
-    CG_TRY(degree_order(graph, p->perm, new_of, nullptr));
+    double share = 1.0;
+    CG_TRY(degree_order(graph, p->perm, new_of, few ? &share : nullptr));
+    if (few && share < kPairShare) {
+      *few = false;
+      return CG_OK;
+    }
     CG_TRY(relabel_graph(graph, new_of.p, &rg));
   }
   const DevGraph g{rg.d_off.p, rg.d_dst.p, nullptr, nullptr, nullptr, V};
@@ -1883,6 +1927,10 @@ int build_pairs(cg_graph* graph, PrPlan* p, hipStream_t s) {
   CG_HIP(hipMemcpyAsync(&P32, incl.p + E - 1, 4, hipMemcpyDeviceToHost, s));
   CG_HIP(hipStreamSynchronize(s));
   const uint64_t P = P32;
+  if (few && (double)P > kPairRate * (double)E) {
+    CG_TRY(hot_bin(graph, nb, few, s));
+    if (!*few) return CG_OK;
+  }
   p->pb_pairs = P;
   // pairs: entry 4 B read, contribution 4 B written and 4 B read; edges:
   // 2 B read (+ 4 B per eight); per vertex a degree and a contribution read,
@@ -2011,8 +2059,8 @@ int pr_plan_create(cg_graph* graph, uint32_t layout, uint32_t seg_log2, uint32_t
   // the two are within box-to-box spread, 0.17-0.20 vs 0.17 ms, and below it
   // the pull wins: 0.10 vs 0.12-0.16 ms at 2^20)
   // and over (source, bin) pairs from 2^24, and on skewed graphs -- a hub of
-  // 16 times the average out-degree, the mark of few pairs per edge -- from
-  // 3 * 2^22 edges on 2^18 vertices (twenty sweeps, ms, against the better of
+  // 16 times the average out-degree, and from 2^22 vertices few pairs (build_pairs)
+  // -- from 3 * 2^22 edges on 2^18 vertices (twenty sweeps, ms, against the better of
   // the two above: R-MAT 18 x 64 1.09 vs 1.10, 20 x 16 1.27 vs 1.46, 21 x 8 1.32 vs
   // 1.70, 21 x 16 1.59 vs 2.95, 22 x 8 1.87 vs 3.26, 22 x 16 3.1 vs 6.9, 23 x 16
   // 5.9 vs 11.3; fewer edges: 20 x 8 1.01 vs 0.73; without hubs, 2^22 vertices
@@ -2025,14 +2073,15 @@ int pr_plan_create(cg_graph* graph, uint32_t layout, uint32_t seg_log2, uint32_t
     if (graph->V >= (1u << 24)) layout = kLayoutPairs;
     else if (skewed && graph->V >= (1u << 18) && graph->E >= 3ull << 22) {
       PrPlan* p = new PrPlan();
-      const int st = build_pairs(graph, p, s);
-      if (st == CG_OK) {
+      bool few = true;
+      const int st = build_pairs(graph, p, s, graph->V >= (1u << 22) ? &few : nullptr);
+      if (st == CG_OK && few) {
         *plan = p;
         return CG_OK;
       }
       delete p;
       // building the pairs takes the most memory: the others may still fit
-      if (st != CG_ERR_OOM) return st;
+      if (st != CG_OK && st != CG_ERR_OOM) return st;
       (void)hipGetLastError();
     }
   }

@@ -133,7 +133,9 @@ typedef struct cg_options {
                                      Automatic: a window size in [1, 30] selects 3, 31 selects 1;
                                      0 (with pr_kernel 0) selects 5 from 2^24 to 2^25 vertices and
                                      on skewed graphs of 3 * 2^22 edges and 2^18 vertices or
-                                     more, 4 from 2^22, else 2 above 65 536 vertices */
+                                     more (from 2^22 vertices on if the pairs are few or the
+                                     destinations skewed too), 4 from 2^22, else 2 above 65 536
+                                     vertices */
   uint32_t relabel;               /* BFS / SSSP: run on an engine-owned copy renumbered by
                                      descending out-degree (results come back in the caller's
                                      ids): 0 automatic (at least 2^21 vertices for SSSP, 2^23
