@@ -513,7 +513,7 @@ static int batch_engine(cg_graph* g, int alg, cg_engine** out) {
       eo.hub_delta = g->max_w / 50 > 1 ? g->max_w / 50 : 1;
     }
     cg_engine* e = nullptr;
-    const int rc = cg_engine_create(g, alg, CG_COORDINATION, 1, &eo, &e);
+    const int rc = engine_create(g, alg, CG_COORDINATION, 1, &eo, false, &e);
     if (rc != CG_OK) return rc;
     slot = std::unique_ptr<cg_engine, void (*)(cg_engine*)>(e, cg_engine_destroy);
   }

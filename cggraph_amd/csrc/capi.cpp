@@ -508,8 +508,10 @@ int cg_partition(const cg_graph* cg, int algorithm, cg_partition_info* info) {
   return cg::plan_partition(g, algorithm, cg::device_memory_bytes(), info, nullptr);
 }
 
-int cg_engine_create(const cg_graph* cg, int algorithm, int engine_type, int use_device_num, const cg_options* opt,
-                     cg_engine** out) {
+}  // extern "C"
+
+int cg::engine_create(const cg_graph* cg, int algorithm, int engine_type, int use_device_num, const cg_options* opt,
+                      bool read, cg_engine** out) {
   clear_error();
   if (!cg || !out) return set_error(CG_ERR_INVALID, "NULL argument");
   if (algorithm < CG_BFS || algorithm > CG_PR) return set_error(CG_ERR_INVALID, "unknown algorithm %d", algorithm);
@@ -639,8 +641,16 @@ int cg_engine_create(const cg_graph* cg, int algorithm, int engine_type, int use
   }
   const uint64_t V = g->V;
   const uint64_t words = (V + 63) / 64 + 1;
-  if (!e->host_only) CG_TRY(e->stage.prepare(V * 4));
+  // a small result's pinned memory lies behind the statistics in hst_map
+  const size_t small = V * 4 <= HostStage::kSmall && !e->host_only ? V * 4 : 0;
+  const size_t small_slots = (small + sizeof(DevStats) - 1) / sizeof(DevStats);
+  // (without the buffer the first copy allocates its own)
+  if (read && !small && !e->host_only && e->stage.prepare(V * 4) != CG_OK) clear_error();
   if (algorithm == CG_PR) {
+    if (small) {
+      CG_TRY(e->hst_map.ensure(small_slots));
+      CG_TRY(e->stage.lend(reinterpret_cast<uint8_t*>(e->hst_map.p), small));
+    }
     CG_TRY(e->rank.ensure(V));
     CG_TRY(e->rank2.ensure(V));
     CG_TRY(e->contrib.ensure(V));
@@ -679,8 +689,9 @@ int cg_engine_create(const cg_graph* cg, int algorithm, int engine_type, int use
     }
     CG_TRY(e->st.ensure(2));
     CG_TRY(e->hst.ensure(3));
-    // two iterations, query done, the level cluster's record
-    CG_TRY(e->hst_map.ensure(4, hipHostMallocMapped | hipHostMallocCoherent));
+    // two iterations, query done, the level cluster's record, a small result
+    CG_TRY(e->hst_map.ensure(4 + small_slots, hipHostMallocMapped | hipHostMallocCoherent));
+    if (small) CG_TRY(e->stage.lend(reinterpret_cast<uint8_t*>(e->hst_map.p + 4), small));
     static_assert(sizeof(ClusterRecord) <= sizeof(DevStats), "the record takes a statistics slot");
     std::memset(e->hst_map.p + 3, 0, sizeof(DevStats));
     e->hst_map_dev = e->hst_map.device_ptr();
@@ -710,6 +721,13 @@ int cg_engine_create(const cg_graph* cg, int algorithm, int engine_type, int use
   }
   *out = e.release();
   return CG_OK;
+}
+
+extern "C" {
+
+int cg_engine_create(const cg_graph* g, int algorithm, int engine_type, int use_device_num, const cg_options* opt,
+                     cg_engine** out) {
+  return engine_create(g, algorithm, engine_type, use_device_num, opt, true, out);
 }
 
 int cg_engine_run(cg_engine* e, uint32_t root, void* out, cg_run_stats* stats) {

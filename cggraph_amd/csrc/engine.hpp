@@ -132,6 +132,10 @@ struct cg_engine {
 };
 
 namespace cg {
+// cg_engine_create.  read false: without the buffer of a first result, for an
+// engine of the library's own that only leaves its values in HBM.
+int engine_create(const cg_graph* g, int algorithm, int engine_type, int use_device_num, const cg_options* opt,
+                  bool read, cg_engine** out);
 int engine_run(cg_engine* e, uint32_t root, cg_run_stats* rs);
 // Waits until every kernel queued on the engine's stream has finished, by
 // polling a record that one more kernel publishes (a stream wait behind short
