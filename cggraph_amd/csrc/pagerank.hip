@@ -10,7 +10,8 @@
 // Four layouts, chosen once per graph (the first three pull over the
 // in-edges, the fourth pushes through destination bins):
 //  plain       one sweep over the transposed graph per iteration, in blocks of
-//              consecutive rows staged through LDS (row blocks, below), or
+//              consecutive rows staged through LDS (row blocks, below; a lane
+//              or a wavefront a row where all are short or all long), or
 //              with rows tiered by in-degree: one lane / one wavefront per row,
 //              rows of 8192+ in-edges cut into 8192-edge chunks.
 //  relabelled  the same sweep over a copy of the CSC whose vertex ids are
@@ -60,6 +61,7 @@ struct PrPlan {
   // rows of kRowEdges and more in chunks of their own
   struct RowBlocks {
     uint32_t n = 0, n_chunks = 0;
+    uint32_t lanes = 0;                    // not 0: no blocks, this many lanes a row (k_pr_each)
     DevBuf<uint32_t> row;                  // first row of each block (n + 1 entries)
     DevBuf<uint32_t> long_row;             // the long rows
     DevBuf<uint32_t> row_chunk, arrived;   // their first chunks (one more entry), chunks done in this sweep
@@ -581,10 +583,22 @@ __global__ void k_row_blocks(const uint64_t* __restrict__ off, uint32_t V, uint3
   }
 }
 
+// The long rows, their number in n[0] and the longest row's edges in n[1].
 __global__ void k_row_long(const uint64_t* __restrict__ off, uint32_t V, uint32_t* __restrict__ list,
                            uint32_t* __restrict__ n) {
-  for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V; v += (uint64_t)gridDim.x * blockDim.x)
-    if (off[v + 1] - off[v] >= kRowEdges) list[atomicAdd(n, 1u)] = (uint32_t)v;
+  uint32_t longest = 0;
+  for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V; v += (uint64_t)gridDim.x * blockDim.x) {
+    const uint64_t d = off[v + 1] - off[v];
+    if (d >= kRowEdges) list[atomicAdd(n, 1u)] = (uint32_t)v;
+    const uint32_t m = d < 0xFFFFFFFFull ? (uint32_t)d : 0xFFFFFFFFu;
+    longest = m > longest ? m : longest;
+  }
+#pragma unroll
+  for (int h = 32; h >= 1; h >>= 1) {
+    const uint32_t m = __shfl_xor(longest, h, 64);
+    longest = m > longest ? m : longest;
+  }
+  if (__lane_id() == 0 && longest) atomicMax(n + 1, longest);
 }
 
 __global__ void k_row_ranges(const uint64_t* __restrict__ off, const uint32_t* __restrict__ list, uint32_t n,
@@ -766,6 +780,35 @@ __global__ __launch_bounds__(kBlock) void k_pr_rows(Csc g, RowView b, const floa
   }
 }
 static_assert(2 * kRowEdges <= 1u << 12 && kRowMax <= 1u << 9 && kBlock == 256, "packed row of a block");
+
+// LANES lanes a row and no staging, for graphs whose rows are all short (1) or
+// all long (64); sums in 64 bits as in the blocks.  Edges in flight per lane, 1 /
+// 2 / 4 with one lane (twenty sweeps, us): one random source a row, 1 M rows 218 /
+// 262 / 290, 3-D lattice of 0.5 M 149 / 140 / 151; 4 / 8 with 64: cliques of 1000
+// 215 / 184, uniform 20 000 x 500 562 / 640, 65 000 x 300 1612 / 1810.
+template <bool LAST, int LANES>
+__global__ __launch_bounds__(kBlock) void k_pr_each(Csc g, const float* __restrict__ contrib, float base, float damping,
+                                                    const uint32_t* __restrict__ perm, float* __restrict__ out) {
+  constexpr int kLoads = LANES == 1 ? 2 : 4;
+  const uint64_t v = (blockIdx.x * (uint64_t)kBlock + threadIdx.x) / LANES;
+  if (v >= g.V) return;  // wave-uniform with 64 lanes a row
+  const uint64_t e = g.off[v + 1];
+  const uint32_t deg = LAST ? 0u : g.deg[v];
+  double sum = 0.0;
+  for (uint64_t k = g.off[v] + threadIdx.x % LANES; k < e; k += kLoads * LANES) {
+    uint32_t u[kLoads];
+    float x[kLoads];
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j) u[j] = ld_src(g.src + (k + j * LANES < e ? k + j * LANES : k));
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j) x[j] = contrib[u[j]];
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j) sum += k + j * LANES < e ? x[j] : 0.0f;
+  }
+#pragma unroll
+  for (int h = LANES / 2; h >= 1; h >>= 1) sum += __shfl_xor(sum, h, LANES);
+  if (threadIdx.x % LANES == 0) row_done<LAST>((uint32_t)v, sum, deg, base, damping, perm, out);
+}
 
 // ---- segmented layout construction ----
 
@@ -952,22 +995,39 @@ bool row_blocks_fit(uint32_t kernel, int layout, uint32_t V, uint64_t E) {
   return E < 3ull << 24 && !(layout == kLayoutPlain && V > (1u << 16) && E < 4ull * V);
 }
 
+// Lanes a row instead of blocks (0: blocks).  One where every row is so short
+// that a lane's chain is shorter than a block's three barriers (twenty sweeps,
+// us, blocks and one lane: paths of 10^3 / 0.3 M / 1 M vertices 105 / 113 / 180 and
+// 92 / 93 / 109, lattices of 65 000 / 0.5 M in 2-D 113 / 182 and 92 / 145, in 3-D
+// 116 / 190 and 94 / 140, four random sources a row, 0.5 M 287 and 260, 1 M 540
+// each).  A wavefront where all rows are so long that a block has one or two, and
+// about as long as each other, so that none holds a wavefront up (cliques of
+// 400 / 500 / 1000, 7.5-10 M edges, 434 / 316 / 435 and 234 / 165 / 215, uniform
+// 20 000 x 500 613 and 562, but 65 000 x 300 1519 and 1612).
+uint32_t row_lanes(uint64_t longest, uint32_t V, uint64_t E) {
+  if (longest <= 2 || (longest <= 6 && V <= (1u << 19))) return 1;
+  return E >= 384ull * V && longest <= 2 * (E / V) ? 64 : 0;
+}
+
 // Row blocks and the chunks of the long rows over a CSC.
 int build_rows(const uint64_t* off, uint32_t V, uint64_t E, PrPlan::RowBlocks& b, hipStream_t s) {
   b.n = (uint32_t)((E + (uint64_t)kRowCost * V + kRowEdges - 1) / kRowEdges);
   CG_TRY(b.row.ensure(b.n + 1));
   const uint64_t max_long = E / kRowEdges;
   DevBuf<uint32_t> cnt;
-  CG_TRY(cnt.ensure(1));
+  CG_TRY(cnt.ensure(2));
   CG_TRY(b.long_row.ensure(max_long ? max_long : 1));
-  CG_HIP(hipMemsetAsync(cnt.p, 0, sizeof(uint32_t), s));
+  CG_HIP(hipMemsetAsync(cnt.p, 0, 2 * sizeof(uint32_t), s));
   hipLaunchKernelGGL(k_row_blocks, dim3(grid_of(b.n + 1)), dim3(kBlock), 0, s, off, V, b.n, b.row.p);
   PR_LAUNCH_OK();
   hipLaunchKernelGGL(k_row_long, dim3(grid_of(V)), dim3(kBlock), 0, s, off, V, b.long_row.p, cnt.p);
   PR_LAUNCH_OK();
-  uint32_t n = 0;
-  CG_HIP(hipMemcpyAsync(&n, cnt.p, sizeof(n), hipMemcpyDeviceToHost, s));
+  uint32_t h[2] = {0, 0};
+  CG_HIP(hipMemcpyAsync(h, cnt.p, sizeof(h), hipMemcpyDeviceToHost, s));
   CG_HIP(hipStreamSynchronize(s));
+  b.lanes = row_lanes(h[1], V, E);
+  if (b.lanes) return CG_OK;
+  const uint32_t n = h[0];
   if (!n) return CG_OK;
   DevBuf<uint64_t> lo, hi;
   CG_TRY(lo.ensure(n));
@@ -2267,14 +2327,20 @@ int pr_run(const DevGraph& g, PrPlan* plan, int iters, float damping, float* ran
       launch_tiers<0>(csc, plan->tiers[0], vblocks, c_cur, base, damping, nullptr, r_nxt, c_nxt, s);
     } else {
       const PrPlan::RowBlocks& b = plan->rows;
-      const RowView view{b.row.p,      b.row_chunk.p, b.long_row.p, b.chunk_of.p, b.chunk_lo.p,
-                         b.chunk_hi.p, b.arrived.p,   b.partial.p,  b.n_chunks};
-      if (it + 1 < iters)
-        hipLaunchKernelGGL(k_pr_rows<false>, dim3(b.n_chunks + b.n), dim3(kBlock), 0, s, csc, view, c_cur, base,
-                           damping, nullptr, c_nxt);
-      else
-        hipLaunchKernelGGL(k_pr_rows<true>, dim3(b.n_chunks + b.n), dim3(kBlock), 0, s, csc, view, c_cur, base,
-                           damping, relabel ? plan->perm.p : nullptr, rank);
+      const bool last = it + 1 == iters;
+      const uint32_t* perm = last && relabel ? plan->perm.p : nullptr;
+      float* out = last ? rank : c_nxt;
+      if (b.lanes) {
+        const dim3 grid((unsigned)(((uint64_t)V * b.lanes + kBlock - 1) / kBlock));
+        hipLaunchKernelGGL(b.lanes == 1 ? (last ? k_pr_each<true, 1> : k_pr_each<false, 1>)
+                                        : (last ? k_pr_each<true, 64> : k_pr_each<false, 64>),
+                           grid, dim3(kBlock), 0, s, csc, c_cur, base, damping, perm, out);
+      } else {
+        const RowView view{b.row.p,      b.row_chunk.p, b.long_row.p, b.chunk_of.p, b.chunk_lo.p,
+                           b.chunk_hi.p, b.arrived.p,   b.partial.p,  b.n_chunks};
+        hipLaunchKernelGGL(last ? k_pr_rows<true> : k_pr_rows<false>, dim3(b.n_chunks + b.n), dim3(kBlock), 0, s, csc,
+                           view, c_cur, base, damping, perm, out);
+      }
     }
     if (profile) {
       CG_HIP(hipEventRecord(b, s));

@@ -143,7 +143,8 @@ typedef struct cg_options {
                                      the edges), 1 never, 2 always */
   uint32_t pr_kernel;             /* PageRank sweep over layouts 1 and 2: 0 automatic (row blocks
                                      below 3 * 2^24 edges -- about 1024 in-edges of consecutive
-                                     rows per workgroup, longer rows in chunks, 64-bit sums --
+                                     rows per workgroup, longer rows in chunks, or a lane / a
+                                     wavefront a row where all are short / long, 64-bit sums --
                                      else row tiers), 1 row tiers (a lane / wavefront /
                                      workgroup per row by in-degree), 2 edge tiles
                                      (2048 consecutive in-edges per workgroup, rows combined by a
