@@ -666,7 +666,7 @@ int cg::engine_create(const cg_graph* cg, int algorithm, int engine_type, int us
     CG_TRY(e->bm[1].ensure(words));
     CG_TRY(e->q_small.ensure(V));
     CG_TRY(e->q_med.ensure(V));
-    uint32_t min_chunk = std::min(e->opt.chunk_edges, chunk_edges_for(g->E));
+    uint32_t min_chunk = std::min(e->opt.chunk_edges, chunk_edges_for(g->E, e->caller_g->max_outdeg));
     // narrow frontiers on the GPU schedule run in a level cluster; traces,
     // profiles and bottom-up min steps are the per-iteration pipeline's
     const bool cluster = e->opt.sched_mode == CG_SCHED_GPU && !e->partial && !e->opt.trace_path && !e->opt.profile &&

@@ -594,7 +594,7 @@ int engine_run(cg_engine* e, uint32_t root, cg_run_stats* rs) {
   Bins fbins{e->opt.bin_wave, e->opt.bin_chunk, e->opt.chunk_edges, e->opt.expand_grid};
   if (mode == CG_SCHED_GPU && fbins.bin_chunk == kBinChunk && fbins.chunk_edges == kChunkEdges) {
     // the default tiers, by the graph's size (chunk_edges_for)
-    fbins.chunk_edges = chunk_edges_for(g.E);
+    fbins.chunk_edges = chunk_edges_for(g.E, e->caller_g->max_outdeg);
     fbins.bin_chunk = std::max(fbins.bin_wave, 2 * fbins.chunk_edges);
   }
   // SSSP's first frontier is the root alone, whose edges go to as many

@@ -46,11 +46,13 @@ constexpr uint32_t kChunkSpread = 2048;
 // (SSSP, 4096 / 2048 -> the rule's: 1 M vertices and 12 M edges 1128 -> 945 us,
 // 200 k / 2.3 M 839 -> 645, R-MAT s20 1523 -> 1299, s22 1942 -> 1809; chunks of
 // 128: 977, 640, 1316, 2075; of 256 at s23 4962 against 4794 of the rule's
-// 1024.  BFS: s14 114 -> 70, s15 104 -> 62, s19 140 -> 135, s22 245 -> 238).
+// 1024.  BFS: s14 114 -> 70, s15 104 -> 62, s19 140 -> 135, s22 245 -> 238).  A
+// vertex is not cut into more than 2 * kChunkSpread chunks, as many as spread a
+// lone one (SSSP on a star of 4 M edges, chunks of 256 464 us, 1024 388).
 constexpr uint32_t kBinChunk = 4096, kChunkEdges = 2048;
-inline uint32_t chunk_edges_for(uint64_t E) {
+inline uint32_t chunk_edges_for(uint64_t E, uint64_t max_outdeg) {
   uint32_t ce = kChunkEdges;
-  while (ce > 256 && E < (uint64_t)ce * 8 * 8192) ce >>= 1;
+  while (ce > 256 && E < (uint64_t)ce * 8 * 8192 && max_outdeg < (uint64_t)ce * kChunkSpread) ce >>= 1;
   return ce;
 }
 
