@@ -31,11 +31,13 @@
 // Queries whose frontiers are narrow do not take part in the levels: a
 // 2048^2 lattice alone drags every other query through its 4500 levels at
 // 20 us.  Level clusters (cluster.hpp) run them root to end, one launch for
-// all, beside the engines and the levels.  52 queries, four on each of R-MAT
+// all, beside the engines and the levels; of the SSSP queries among them
+// whose frontiers are wide, as many as end sooner on engines run there
+// (batch_wide_on_cluster).  52 queries, four on each of R-MAT
 // s14-s22 and lattices of 256^2-2048^2: 126 -> 71 ms, the cluster launch 41
-// ms of it (54.5 with the results copied while engines run); with every query of the 512-query set off the engines 328 -> 215
-// ms; with the s18-s22 queries on engines that set is bound by the engine
-// thread and stays at 237 ms.
+// ms of it (54.5 with the results copied while engines run); with every query
+// of the 512-query set off the engines 328 -> 215 ms; with the s18-s22 queries
+// on engines that set is bound by the engine thread (237 ms, 219 since).
 //
 // The relaxation is the reference's (my_project/CGgraph/device_algorithm.cuh:
 // 51-54 BFS, 253-257 SSSP), so each query ends at its unique fixed point,
